@@ -245,7 +245,7 @@ int fm_router_logits(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64_
  * of 512 with the gate [8, D] in 64 KiB (D <= 2048 for an fp32 gate, <= 4096
  * for a bf16 one) the gate, gating, loss partials and counts run as one pass
  * over x plus one small kernel (fm_router_forward_fused says which); other
- * shapes launch the steps separately.  T > 0; the workspace holds
+ * gates with bf16 x take three launches, fp32 x the steps separately.  T > 0; the workspace holds
  * fm_router_forward_workspace_bytes(T, E) bytes. */
 int64_t fm_router_forward_workspace_bytes(int64_t T, int E);
 int fm_router_forward_fused(int E, int64_t D, int w_dtype);
@@ -308,7 +308,8 @@ int fm_gating_grad_dot(const float* logits, int64_t T, int E, int64_t ld_l, int 
  * autograd): dx = dlogits w (x's dtype, null to skip; w fp32 or bf16),
  * dw = dlogits^T x and db = sum_t dlogits (fp32 sums, null to skip, written
  * as dw_dtype / db_dtype), summed in a fixed order; dw and db need a
- * workspace of fm_router_workspace_bytes(T, D, E) bytes. */
+ * workspace of fm_router_workspace_bytes(T, D, E) bytes, and dx alone is faster
+ * with one (bf16 x, E > 8: the matrix cores). */
 int64_t fm_router_workspace_bytes(int64_t T, int64_t D, int E);
 int fm_router_backward(const float* dlogits, int64_t ld_dl, const void* x, int x_dtype, int64_t ld_x, int64_t T,
                        int64_t D, const void* w, int w_dtype, int64_t ld_w, int E, void* dx, int64_t ld_dx, void* dw,

@@ -113,4 +113,33 @@ __device__ __forceinline__ int gate_group(const GateOut& a, int64_t t, bool tv, 
   return my_i;
 }
 
+// What the gating kernels of fm_topk_gating read and write; with `part` (the
+// router forward) the logits come as S chunk sums, bias and score bias are
+// added here, and the partials are per workgroup and expert-major.
+struct TopkArgs {
+  const float* logits;   // [T, E] row pitch ld
+  int64_t T, ld;
+  int E, K;
+  int sigmoid;
+  int l2;                // normalise the K weights by their l2 norm (+1e-8)
+  const void* replay;    // [T, K] experts to replay (R3), or null
+  int replay_i64;
+  float* w;              // [T, K]
+  void* idx;             // [T, K] int64 or int32
+  int idx_i64;
+  float* prob_partial;   // [n_waves, E] or null: per-wave sums of softmax(logits); router: [E, workgroups]
+  float* z_partial;      // [n_waves] or null: per-wave sums of logsumexp(logits)^2; router: [workgroups]
+  const float* part;     // router: [S][T][ld_p] chunk sums of the gate
+  int64_t S, ld_p;
+  const void* bias;      // [E] or null
+  int bias_bf16;
+  const float* score_bias;   // [E] or null
+  float* logits_out;     // [T, ld]
+  int32_t* hist;         // [E, workgroups]: routed slots
+};
+// Gating of the router forward for E > 8 or a gate outside the small-gate
+// kernel (defined beside the gating kernels): nb workgroups of kRouterGateWaves waves.
+constexpr int kRouterGateWaves = 16;
+int router_gate_launch(const TopkArgs& a, int64_t nb, hipStream_t s, const char* what);
+
 }  // namespace fm

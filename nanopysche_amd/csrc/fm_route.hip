@@ -28,37 +28,116 @@
 namespace fm {
 
 // ---------------------------------------------------------------- top-k ----
-struct TopkArgs {
-  const float* logits;   // [T, E] row pitch ld
-  int64_t T, ld;
-  int E, K;
-  int sigmoid;
-  int l2;                // normalise the K weights by their l2 norm (+1e-8)
-  const void* replay;    // [T, K] experts to replay (R3), or null
-  int replay_i64;
-  float* w;              // [T, K]
-  void* idx;             // [T, K] int64 or int32
-  int idx_i64;
-  float* prob_partial;   // [n_waves, E] or null: per-wave sums of softmax(logits)
-  float* z_partial;      // [n_waves] or null: per-wave sums of logsumexp(logits)^2
-};
-
 constexpr int kTopkMaxPerLane = 4;  // E <= 256
 
+// The logits of experts e + 64 j (j < NJ) of token t (-inf from E on): read, or
+// (ROUTER) the gate's chunk sums added in chunk order, plus bias and score
+// bias, and written.  Eight chunks' loads of every j are in flight at once.
+template <bool ROUTER, int NJ>
+__device__ __forceinline__ void topk_logits(const TopkArgs& a, int64_t t, int e, float (&v)[NJ]) {
+  if constexpr (!ROUTER) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) v[j] = e + 64 * j < a.E ? a.logits[t * a.ld + e + 64 * j] : -INFINITY;
+  } else {
+    const float* p = a.part + t * a.ld_p;
+    const int64_t plane = a.T * a.ld_p;
+    int c[NJ];   // experts past E read the last one
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) c[j] = e + 64 * j < a.E ? e + 64 * j : a.E - 1;
+    for (int64_t s = 0; s < a.S; s += 8) {
+      float u[8][NJ];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) u[i][j] = p[(s + i < a.S ? s + i : s) * plane + c[j]];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (s + i < a.S)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) v[j] = s + i == 0 ? u[0][j] : v[j] + u[i][j];
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (a.bias)
+        v[j] += a.bias_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(a.bias)[c[j]]) : static_cast<const float*>(a.bias)[c[j]];
+      if (a.score_bias) v[j] += a.score_bias[c[j]];
+      if (e + 64 * j < a.E) a.logits_out[t * a.ld + e + 64 * j] = v[j];
+      else v[j] = -INFINITY;
+    }
+  }
+}
+
+// Largest of the 64 lanes' values, in every lane (DPP: a few cycles a step,
+// where a shuffle is an LDS round trip).
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+  auto step = [&](auto ctrl, auto rows) {
+    const uint32_t o = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+    v = o > v ? o : v;
+  };
+  step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr 1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast 15, 31
+  step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+  return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+
+// An unsigned key in the selection order of `beats`: NaN above every number,
+// then larger; -0 and +0 alike.  Never 0.
+__device__ __forceinline__ uint32_t score_key(float v) {
+  const uint32_t u = v == 0.f ? 0u : f2u(v);
+  return v != v ? 0xffffffffu : (u & 0x80000000u) ? ~u : u | 0x80000000u;
+}
+
+// Per-workgroup partials of the router forward: the waves' softmax and
+// logsumexp^2 sums in wave order, and the histogram of the routed slots.
+struct RouterPartials {
+  float p[kRouterGateWaves][64 * kTopkMaxPerLane];
+  float z[kRouterGateWaves];
+  int32_t hist[64 * kTopkMaxPerLane];
+};
+__device__ __forceinline__ void write_router_partials(const TopkArgs& a, const RouterPartials& r) {
+  const int64_t nb = gridDim.x;
+  const int e = threadIdx.x;
+  if (e < a.E) {
+    float p = r.p[0][e];
+#pragma unroll
+    for (int w = 1; w < kRouterGateWaves; ++w) p += r.p[w][e];
+    a.hist[e * nb + blockIdx.x] = r.hist[e];
+    a.prob_partial[e * nb + blockIdx.x] = p;
+  }
+  if (a.z_partial && e == 0) {
+    float z = r.z[0];
+    for (int w = 1; w < kRouterGateWaves; ++w) z += r.z[w];
+    a.z_partial[blockIdx.x] = z;
+  }
+}
+
 // One token per wave; lane l holds experts l + 64 j.  Each of the K rounds is
-// a wave arg-max over the experts not yet taken (a per-lane taken mask, so an
-// expert never wins twice even when every remaining score is -inf).
+// a wave arg-max over the experts not yet taken (a taken expert's key is 0,
+// below every other, so an expert never wins twice even when every remaining
+// score is -inf): the largest key by DPP, then the lowest expert that holds it
+// from one ballot per j.  (With shuffles of value and index the rounds were
+// dependent LDS round trips: 42 us for [4096, 256], K = 8; now 7.)
 //   softmax:  top-k of the logits, w = softmax over the K selected logits
 //   sigmoid:  top-k of sigmoid(logits), w = s / (sum s + 1e-8)
 //   replay:   p = softmax(all logits), w_e = p_e / max(sum over the replayed
 //             experts of p, 1e-8) on the replayed experts and 0 elsewhere;
 //             the K largest w in order (the reference's R3 gating)
 // then optionally w / (||w||_2 + 1e-8).
-__global__ __launch_bounds__(256) void topk_kernel(TopkArgs a) {
+template <bool ROUTER>
+__global__ __launch_bounds__(ROUTER ? 64 * kRouterGateWaves : 256) void topk_kernel(TopkArgs a) {
+  constexpr int kWaves = ROUTER ? kRouterGateWaves : 4;
+  __shared__ RouterPartials part;
   const int lane = threadIdx.x & 63;
-  const int64_t wave = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int64_t n_waves = int64_t(gridDim.x) * 4;
+  const int64_t wave = int64_t(blockIdx.x) * kWaves + (threadIdx.x >> 6);
+  const int64_t n_waves = int64_t(gridDim.x) * kWaves;
   const bool need_p = a.prob_partial || a.replay || a.z_partial;
+  if constexpr (ROUTER) {
+    if (threadIdx.x < 64 * kTopkMaxPerLane) part.hist[threadIdx.x] = 0;
+    __syncthreads();
+  }
   float psum[kTopkMaxPerLane];
 #pragma unroll
   for (int j = 0; j < kTopkMaxPerLane; ++j) psum[j] = 0.f;
@@ -66,12 +145,9 @@ __global__ __launch_bounds__(256) void topk_kernel(TopkArgs a) {
   for (int64_t t = wave; t < a.T; t += n_waves) {
     float v[kTopkMaxPerLane];   // logits of experts lane + 64*j
     float sc[kTopkMaxPerLane];  // selection scores
+    topk_logits<ROUTER>(a, t, lane, v);
 #pragma unroll
-    for (int j = 0; j < kTopkMaxPerLane; ++j) {
-      const int e = lane + 64 * j;
-      v[j] = e < a.E ? a.logits[t * a.ld + e] : -INFINITY;
-      sc[j] = a.sigmoid ? 1.f / (1.f + expf(-v[j])) : v[j];
-    }
+    for (int j = 0; j < kTopkMaxPerLane; ++j) sc[j] = a.sigmoid ? 1.f / (1.f + expf(-v[j])) : v[j];
     if (need_p) {
       float m = -INFINITY;
 #pragma unroll
@@ -108,33 +184,41 @@ __global__ __launch_bounds__(256) void topk_kernel(TopkArgs a) {
         for (int j = 0; j < kTopkMaxPerLane; ++j) sc[j] /= msum;
       }
     }
-    uint32_t taken = 0;
+    uint32_t key[kTopkMaxPerLane];
+#pragma unroll
+    for (int j = 0; j < kTopkMaxPerLane; ++j) key[j] = lane + 64 * j < a.E ? score_key(sc[j]) : 0u;
     float top_first = 0.f, wsum = 0.f, my_w = 0.f;
     int my_i = 0;
     for (int k = 0; k < a.K; ++k) {
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
+      uint32_t best = key[0];
+#pragma unroll
+      for (int j = 1; j < kTopkMaxPerLane; ++j) best = key[j] > best ? key[j] : best;
+      best = wave_umax(best);
+      // the lowest expert with that key: K <= E candidates exist in every round
+      int jw = 0, lw = 0;
+      bool found = false;
 #pragma unroll
       for (int j = 0; j < kTopkMaxPerLane; ++j) {
-        const int e = lane + 64 * j;
-        if (e < a.E && !((taken >> j) & 1u) && beats(sc[j], e, bv, bi)) { bv = sc[j]; bi = e; }
+        const uint64_t mask = __ballot(key[j] == best);
+        if (!found && mask != 0) {
+          found = true;
+          jw = j;
+          lw = __builtin_ctzll(mask);
+        }
       }
-      for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(bv, off);
-        const int oi = __shfl_xor(bi, off);
-        if (beats(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-      }
-      const int jw = bi >> 6;   // bi < E: K <= E candidates exist in every round
-      if ((bi & 63) == lane) taken |= 1u << jw;
-      float vj = v[0];
+      float vj = v[0], sj = sc[0];
 #pragma unroll
-      for (int j = 1; j < kTopkMaxPerLane; ++j) vj = jw == j ? v[j] : vj;
-      const float lg = __shfl(vj, bi & 63);
+      for (int j = 0; j < kTopkMaxPerLane; ++j) {
+        if (jw == j) { vj = v[j]; sj = sc[j]; }
+        if (jw == j && lane == lw) key[j] = 0u;
+      }
+      const float lg = u2f(uint32_t(__builtin_amdgcn_readlane(int(f2u(vj)), lw)));
+      const float bv = u2f(uint32_t(__builtin_amdgcn_readlane(int(f2u(sj)), lw)));
       if (k == 0) top_first = lg;
       // sigmoid and replay weights are the scores; softmax: exp(l - l_max)
       const float wk = (a.sigmoid || a.replay) ? bv : expf(lg - top_first);
       wsum += wk;
-      if (lane == k) { my_w = wk; my_i = bi; }
+      if (lane == k) { my_w = wk; my_i = lw + 64 * jw; }
     }
     float wn = a.replay ? my_w : (a.sigmoid ? my_w / (wsum + 1e-8f) : my_w / wsum);
     if (a.l2) {
@@ -145,48 +229,93 @@ __global__ __launch_bounds__(256) void topk_kernel(TopkArgs a) {
     if (lane < a.K) {
       a.w[t * a.K + lane] = wn;
       store_index(a.idx, a.idx_i64, t * a.K + lane, my_i);
+      if constexpr (ROUTER) atomicAdd(&part.hist[my_i], 1);
     }
   }
-  if (a.prob_partial) {
+  if constexpr (ROUTER) {
+    const int w4 = threadIdx.x >> 6;
 #pragma unroll
-    for (int j = 0; j < kTopkMaxPerLane; ++j) {
-      const int e = lane + 64 * j;
-      if (e < a.E) a.prob_partial[wave * a.E + e] = psum[j];
+    for (int j = 0; j < kTopkMaxPerLane; ++j) part.p[w4][lane + 64 * j] = psum[j];
+    if (lane == 0) part.z[w4] = zsum;
+    __syncthreads();
+    write_router_partials(a, part);
+  } else {
+    if (a.prob_partial) {
+#pragma unroll
+      for (int j = 0; j < kTopkMaxPerLane; ++j) {
+        const int e = lane + 64 * j;
+        if (e < a.E) a.prob_partial[wave * a.E + e] = psum[j];
+      }
     }
+    if (a.z_partial && lane == 0) a.z_partial[wave] = zsum;
   }
-  if (a.z_partial && lane == 0) a.z_partial[wave] = zsum;
 }
 
 // E <= 16: a wave takes 64 / EP tokens at once (EP = E rounded up to a power
 // of two; lane = token slot * EP + expert), so the reductions run over EP
 // lanes (log2 EP steps) for NT tokens together instead of over 64 lanes for
 // one token.  Same selection rule, weights (sum over k in k order), replay,
-// l2 normalisation and per-wave partials as topk_kernel.
-template <int EP>
-__global__ __launch_bounds__(256) void topk_small_kernel(TopkArgs a) {
-  constexpr int NT = 64 / EP;
+// l2 normalisation and partials as topk_kernel.
+template <int EP, bool ROUTER>
+__global__ __launch_bounds__(ROUTER ? 64 * kRouterGateWaves : 256) void topk_small_kernel(TopkArgs a) {
+  constexpr int NT = 64 / EP, kWaves = ROUTER ? kRouterGateWaves : 4;
+  __shared__ RouterPartials part;
   const int lane = threadIdx.x & 63, g = lane / EP, e = lane % EP;
-  const int64_t wave = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int64_t n_waves = int64_t(gridDim.x) * 4;
+  const int64_t wave = int64_t(blockIdx.x) * kWaves + (threadIdx.x >> 6);
+  const int64_t n_waves = int64_t(gridDim.x) * kWaves;
   const GateOut go{a.E, a.K, a.sigmoid, a.l2, a.replay, a.replay_i64, a.w, a.idx, a.idx_i64,
                    (a.prob_partial || a.replay || a.z_partial) ? 1 : 0};
+  if constexpr (ROUTER) {
+    if (threadIdx.x < 64 * kTopkMaxPerLane) part.hist[threadIdx.x] = 0;
+    __syncthreads();
+  }
   float psum = 0.f, zsum = 0.f;
   for (int64_t tg = wave; tg * NT < a.T; tg += n_waves) {
     const int64_t t = tg * NT + g;
     const bool tv = t < a.T;
-    const float v = (tv && e < a.E) ? a.logits[t * a.ld + e] : -INFINITY;
-    gate_group<EP>(go, t, tv, g, e, v, psum, zsum);
+    float v[1] = {-INFINITY};
+    if (tv) topk_logits<ROUTER>(a, t, e, v);
+    const int my_i = gate_group<EP>(go, t, tv, g, e, v[0], psum, zsum);
+    if constexpr (ROUTER)
+      if (tv && e < a.K) atomicAdd(&part.hist[my_i], 1);
   }
-  if (a.prob_partial) {
+  if (ROUTER || a.prob_partial) {
 #pragma unroll
     for (int off = EP; off < 64; off <<= 1) psum += __shfl_xor(psum, off);
-    if (lane < a.E) a.prob_partial[wave * a.E + lane] = psum;
+    if constexpr (ROUTER) {
+      if (lane < a.E) part.p[threadIdx.x >> 6][lane] = psum;
+    } else {
+      if (lane < a.E) a.prob_partial[wave * a.E + lane] = psum;
+    }
   }
   if (a.z_partial) {
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) zsum += __shfl_xor(zsum, off);
-    if (lane == 0) a.z_partial[wave] = zsum;
+    if constexpr (ROUTER) {
+      if (lane == 0) part.z[threadIdx.x >> 6] = zsum;
+    } else {
+      if (lane == 0) a.z_partial[wave] = zsum;
+    }
   }
+  if constexpr (ROUTER) {
+    __syncthreads();
+    write_router_partials(a, part);
+  }
+}
+
+template <bool ROUTER>
+int topk_launch(const TopkArgs& a, int64_t nb, hipStream_t s, const char* what) {
+  const dim3 grid{unsigned(nb)}, block{ROUTER ? 64 * kRouterGateWaves : 256};
+  if (a.E <= 2) hipLaunchKernelGGL((topk_small_kernel<2, ROUTER>), grid, block, 0, s, a);
+  else if (a.E <= 4) hipLaunchKernelGGL((topk_small_kernel<4, ROUTER>), grid, block, 0, s, a);
+  else if (a.E <= 8) hipLaunchKernelGGL((topk_small_kernel<8, ROUTER>), grid, block, 0, s, a);
+  else if (a.E <= 16) hipLaunchKernelGGL((topk_small_kernel<16, ROUTER>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL(topk_kernel<ROUTER>, grid, block, 0, s, a);
+  return check_launch(what);
+}
+
+int router_gate_launch(const TopkArgs& a, int64_t nb, hipStream_t s, const char* what) {
+  return topk_launch<true>(a, nb, s, what);
 }
 
 // one block of 512 threads: wave w sums experts w, w + 8, ... -- each lane a
@@ -1135,14 +1264,7 @@ int fm_topk_gating(const float* logits, int64_t T, int E, int64_t ld, int K, int
   if (T == 0) return 0;
   TopkArgs a{logits, T, ld, E, K, gating == FM_GATING_SIGMOID, (flags & FM_GATING_L2_NORMALIZE) ? 1 : 0,
              replay_indices, replay_i64, weights, indices, indices_i64, prob_partial, z_partial};
-  const dim3 grid(unsigned(n_waves / 4)), block(256);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (E <= 2) hipLaunchKernelGGL(topk_small_kernel<2>, grid, block, 0, s, a);
-  else if (E <= 4) hipLaunchKernelGGL(topk_small_kernel<4>, grid, block, 0, s, a);
-  else if (E <= 8) hipLaunchKernelGGL(topk_small_kernel<8>, grid, block, 0, s, a);
-  else if (E <= 16) hipLaunchKernelGGL(topk_small_kernel<16>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(topk_kernel, grid, block, 0, s, a);
-  return check_launch("fm_topk_gating");
+  return topk_launch<false>(a, n_waves / 4, static_cast<hipStream_t>(stream), "fm_topk_gating");
 }
 
 int fm_aux_loss(const float* prob_partial, int64_t n_waves, const int32_t* counts, int E, int64_t T,

@@ -2,8 +2,9 @@
 //   fm_router_forward    the whole forward of the router in two launches for small gates
 //                        (E <= 8, D = 512 n <= 2048): logits, top-k gating, the softmax
 //                        and logsumexp^2 partials and per-workgroup expert histograms in
-//                        one pass over x, then counts + load-balancing (+ z) loss; other
-//                        shapes run the same steps as separate kernels
+//                        one pass over x, then counts + load-balancing (+ z) loss; in three
+//                        for other gates with bf16 x (the gate's chunk sums, gating and
+//                        partials, counts + loss); fp32 x runs the steps as separate kernels
 //   fm_router_logits     logits[t][e] = sum_d x[t][d] * w[e][d] + bias[e] + score_bias[e], fp32
 //                        (the reference's gate(x.float()) + score_bias, :151-154)
 //   fm_expert_counts     counts[e] = number of the T*K slots routed to e (the f_i of the
@@ -19,13 +20,14 @@
 //
 // The gate is a skinny GEMM (E <= 256 outputs per token): x is read once at
 // its size and the products are summed in fp32, as the reference computes
-// it -- on the matrix cores for bf16 x and a bf16 gate with E <= 8, D <= 2048
-// (bf16 products are exact in fp32; the order of the sums differs), otherwise
-// as FMAs on the VALU; HBM, not arithmetic, bounds it at the layer's shapes.
+// it -- on the matrix cores for bf16 x (bf16 products are exact in fp32, an fp32
+// gate is three exact bf16 pieces, fm_router_mfma.h; the order of the sums
+// differs) except for a small fp32 gate, otherwise as FMAs on the VALU.
 // Gate weights are read as stored (fp32 or bf16).
 #include <type_traits>
 
 #include "fm_gating.h"
+#include "fm_router_mfma.h"
 #include "../../include/fm_hip.h"
 
 namespace fm {
@@ -252,9 +254,6 @@ struct RouterFuse {
   float* z_partial;      // [gridDim.x] or null
   int32_t* block_hist;   // [E, gridDim.x]
 };
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 // bf16 x and gate, D <= 2048: the workgroup's 16 x 8 logits as one 16x16
 // MFMA tile (tokens x experts, experts 8..15 zero), wave w contracting its
@@ -511,6 +510,72 @@ __global__ __launch_bounds__(576) void router_finish_kernel(const int32_t* block
   }
 }
 
+// The same after the gating kernel of the other gates (bf16 x): 16 waves, an
+// expert each at a time, nb <= 256 workgroups' partials in one 4-entry read per lane.
+__global__ __launch_bounds__(1024) void router_finish_wide_kernel(const int32_t* block_hist, int64_t nb, int E,
+                                                                  int32_t* counts, int64_t* acc, int64_t* acc_total,
+                                                                  int64_t T, const float* prob_partial,
+                                                                  const float* z_partial, float z_mult, float* loss) {
+  __shared__ float term[256];
+  __shared__ float zterm;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto row = [&](const float* r, float (&v)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = lane + 64 * u < nb ? r[lane + 64 * u] : 0.f;
+  };
+  auto sum4 = [](const float (&v)[4]) { return ((v[0] + v[1]) + v[2]) + v[3]; };
+  for (int e0 = wave; e0 < E; e0 += 128) {   // eight experts' loads in flight
+    float p[8][4];
+    int c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e = e0 + 16 * i < E ? e0 + 16 * i : E - 1;
+      row(prob_partial + int64_t(e) * nb, p[i]);
+      const int32_t* h = block_hist + int64_t(e) * nb;
+      c[i] = 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[i] += lane + 64 * u < nb ? h[lane + 64 * u] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float ps = sum4(p[i]);
+      int cs = c[i];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        cs += __shfl_xor(cs, off);
+        ps += __shfl_xor(ps, off);
+      }
+      const int e = e0 + 16 * i;
+      if (lane == 0 && e < E) {
+        counts[e] = cs;
+        if (acc) acc[e] += cs;
+        term[e] = (float(cs) / float(T)) * (ps / float(T));
+      }
+    }
+  }
+  if (wave == 15 && z_partial) {
+    float v[4];
+    row(z_partial, v);
+    float z = sum4(v);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) z += __shfl_xor(z, off);
+    if (lane == 0) zterm = z / float(T);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float s = 0.f;
+    for (int e = lane; e < E; e += 64) s += term[e];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) {
+      if (acc_total) acc_total[0] += T;
+      float l = float(E) * s;
+      if (z_partial) l = l + z_mult * zterm;
+      loss[0] = l;
+    }
+  }
+}
+
 // --------------------------------------------------------------- counts ----
 // One workgroup: LDS histogram over all T*K slots (fixed E <= 1024 bins).
 // With `acc` the counts are also added to the running per-expert totals and
@@ -758,7 +823,7 @@ struct RouterBwdArgs {
   int64_t slices, rows_per_slice;
 };
 
-// dx: grid (T / 16); wave v rows 16 b + 4 v .. +4, lane l columns 8 l .. of
+// Short rows of at most 8 experts, or fp32 x.  dx: grid (T / 16); wave v rows 16 b + 4 v .. +4, lane l columns 8 l .. of
 // each 512-column chunk, sum over all experts in chunks of 16.
 template <typename T>
 __global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs a) {
@@ -971,6 +1036,32 @@ inline bool router_small_ok(int E, int64_t D, int w_bf16) {
   return E <= 8 && D % kRouterCols == 0 && 8 * D * (w_bf16 ? 2 : 4) <= kGateLdsBytes;
 }
 
+// bf16 x: the gate on the matrix cores, as chunk sums (SPLIT: out = part) or logits.
+template <bool SPLIT>
+int gate_logits_launch(const RouterArgs& r, float* out, int64_t ld_o, hipStream_t s, const char* what) {
+  const GateShape g = gate_shape(r.T, r.D, r.E, !r.w_bf16);
+  const GateLogitsArgs a{static_cast<const uint16_t*>(r.x), r.ld_x, r.T, r.D, r.w, r.ld_w, r.bias, r.score_bias, r.E,
+                         g.S, g.chunk, g.eg, int(g.tt), out, ld_o};
+  const int64_t waves = g.tt * g.eg * (SPLIT ? g.S : 1);
+  const dim3 grid{unsigned((waves + 3) / 4)}, block{256};
+#define FM_GATE(TF, NF, W) hipLaunchKernelGGL((gate_logits_kernel<TF, NF, W, SPLIT>), grid, block, 0, s, a)
+#define FM_GATE_NF(TF, W)              \
+  switch (g.nf) {                      \
+    case 1: FM_GATE(TF, 1, W); break;  \
+    case 2: FM_GATE(TF, 2, W); break;  \
+    case 3: FM_GATE(TF, 3, W); break;  \
+    default: FM_GATE(TF, 4, W); break; \
+  }
+  if (r.w_bf16) {
+    if (g.tf == 1) FM_GATE_NF(1, false) else if (g.tf == 2) FM_GATE_NF(2, false) else FM_GATE_NF(4, false)
+  } else {
+    if (g.tf == 1) FM_GATE_NF(1, true) else FM_GATE_NF(2, true)
+  }
+#undef FM_GATE_NF
+#undef FM_GATE
+  return check_launch(what);
+}
+
 int router_logits_launch(const RouterArgs& a, int x_dtype, const RouterFuse* f, int fused, hipStream_t s,
                          const char* what) {
   const unsigned rb = unsigned((a.T + kRouterRows - 1) / kRouterRows);
@@ -989,16 +1080,22 @@ int router_logits_launch(const RouterArgs& a, int x_dtype, const RouterFuse* f, 
       else { if (xb) FM_SMALL(uint16_t, float, false); else FM_SMALL(float, float, false); }
     }
 #undef FM_SMALL
+  } else if (xb) {
+    return gate_logits_launch<false>(a, a.logits, a.ld_l, s, what);
   } else if (a.E <= 8) {
-    const dim3 grid(rb, 1);
-    if (xb) hipLaunchKernelGGL((router_logits_kernel<uint16_t, 8>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((router_logits_kernel<float, 8>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((router_logits_kernel<float, 8>), dim3(rb, 1), dim3(256), 0, s, a);
   } else {
-    const dim3 grid(rb, unsigned((a.E + 15) / 16));
-    if (xb) hipLaunchKernelGGL((router_logits_kernel<uint16_t, 16>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((router_logits_kernel<float, 16>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((router_logits_kernel<float, 16>), dim3(rb, unsigned((a.E + 15) / 16)), dim3(256), 0, s, a);
   }
   return check_launch(what);
+}
+
+// Workgroups of the router forward's gating kernel (kRouterGateWaves waves, a token
+// or group of tokens per wave and turn; router_finish_wide_kernel reads at most
+// 256 partials per expert).
+inline int64_t gate_blocks(int64_t T) {
+  const int64_t n = (T + kRouterGateWaves - 1) / kRouterGateWaves;
+  return n < 256 ? n : 256;
 }
 
 // slices of the token range for the dw partials: at most 128, and at most
@@ -1009,6 +1106,45 @@ inline int64_t router_slices(int64_t T, int64_t D, int E) {
   s = s < 1 ? 1 : s;
   const int64_t per = (T + s - 1) / s;
   return per > 0 ? (T + per - 1) / per : 1;
+}
+
+int router_backward_mfma(const float* dl, int64_t ld_dl, const void* x, int64_t ld_x, int64_t T, int64_t D,
+                         const void* w, int w_bf16, int64_t ld_w, int E, void* dx, int64_t ld_dx, void* dw, int dw_bf16,
+                         int64_t ld_dw, void* db, int db_bf16, void* workspace, hipStream_t s) {
+  const GateBwdShape g = gate_bwd_shape(T, D, E);
+  uint8_t* base = static_cast<uint8_t*>(workspace);
+  auto at = [&](int64_t off) { return reinterpret_cast<uint16_t*>(base + off); };
+  float* part = reinterpret_cast<float*>(base + g.part);
+  float* db_part = reinterpret_cast<float*>(base + g.db);
+  const uint16_t* xb = static_cast<const uint16_t*>(x);
+  GatePieceArgs pa{dl, ld_dl, T, D, g.Tp, g.Dp, E, g.Ep, w, ld_w, w_bf16, dx ? at(g.p) : nullptr, dw ? at(g.pt) : nullptr,
+                   db ? db_part : nullptr, dx ? at(g.wt) : nullptr, g.t_tiles, dx ? (D + 63) / 64 : 0};
+  hipLaunchKernelGGL(gate_pieces_kernel, dim3(unsigned(pa.t_tiles + pa.d_tiles), unsigned((g.Ep + 63) / 64)),
+                     dim3(256), 0, s, pa);
+  if (int rc = check_launch("fm_router_backward")) return rc;
+  if (dx != nullptr) {
+    const GateDxArgs a{at(g.p), at(g.wt), T, D, g.Tp, g.Dp, g.Ep, static_cast<uint16_t*>(dx), ld_dx};
+    const dim3 grid(unsigned((T + 127) / 128), unsigned((D + 127) / 128));
+    if (w_bf16) hipLaunchKernelGGL(gate_dx_kernel<false>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(gate_dx_kernel<true>, grid, dim3(256), 0, s, a);
+    if (int rc = check_launch("fm_router_backward")) return rc;
+  }
+  if (dw != nullptr) {
+    const GateDwArgs a{at(g.pt), g.Tp, E, g.Ep, xb, ld_x, T, D, g.rows, g.slices, part};
+    const dim3 grid(unsigned((D + 512 / g.we - 1) / (512 / g.we) * g.slices));
+    if (g.we == 1) hipLaunchKernelGGL(gate_dw_kernel<1>, grid, dim3(256), 0, s, a);
+    else if (g.we == 2) hipLaunchKernelGGL(gate_dw_kernel<2>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(gate_dw_kernel<4>, grid, dim3(256), 0, s, a);
+    if (int rc = check_launch("fm_router_backward")) return rc;
+  }
+  if (dw != nullptr || db != nullptr) {
+    const int vec = ld_dw % 4 == 0 && reinterpret_cast<uintptr_t>(dw) % (dw_bf16 ? 8 : 16) == 0;
+    const GateDwSumArgs a{part, g.slices, D, E, dw, ld_dw, dw_bf16, vec, db_part, g.t_tiles, db, db_bf16};
+    const unsigned blocks = dw ? unsigned((D + 1023) / 1024) + 1 : 1;
+    hipLaunchKernelGGL(gate_dw_sum_kernel, dim3(blocks, unsigned(E)), dim3(256), 0, s, a);
+    return check_launch("fm_router_backward");
+  }
+  return 0;
 }
 
 }  // namespace fm
@@ -1037,7 +1173,16 @@ int64_t fm_router_forward_workspace_bytes(int64_t T, int E) {
   const int64_t nb = (T + kRouterRows - 1) / kRouterRows;
   const int64_t fused = nb * (int64_t(E) + 1) * 4 + nb * int64_t(E) * 4;
   const int64_t plain = kRouterForwardWaves * (int64_t(E) + 1) * 4;
-  return fused > plain ? fused : plain;
+  int64_t most = fused > plain ? fused : plain;
+  if (E <= 256) {
+    const int64_t gb = gate_blocks(T);
+    for (int w32 = 0; w32 < 2; ++w32) {   // the chunk sums and the gating kernel's partials, whatever D is
+      const GateShape g = gate_shape(T, 0, E, w32 != 0);
+      const int64_t b = (g.S * T * g.ld_p + gb * (2 * int64_t(E) + 1)) * 4;
+      most = b > most ? b : most;
+    }
+  }
+  return most;
 }
 
 int fm_router_forward_fused(int E, int64_t D, int w_dtype) {
@@ -1083,7 +1228,31 @@ int fm_router_forward(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64
                        total_tokens, T, part, zm != 0.f ? zpart : nullptr, zm, loss);
     return check_launch("fm_router_forward");
   }
-  // other shapes: logits, then gating, counts and loss as separate kernels
+  // other gates with bf16 x: the gate's chunk sums, the gating (which adds them),
+  // and counts + loss
+  if (x_dtype == FM_DTYPE_BF16) {
+    const GateShape g = gate_shape(T, D, E, w_dtype != FM_DTYPE_BF16);
+    const int64_t gb = gate_blocks(T);
+    float* prob = base + g.S * T * g.ld_p;
+    float* zp = prob + gb * E;
+    int32_t* hist = reinterpret_cast<int32_t*>(zp + gb);
+    if (int rc = gate_logits_launch<true>(a, base, g.ld_p, s, "fm_router_forward")) return rc;
+    TopkArgs t{nullptr, T, ld_l, E, K, sigmoid, l2, replay_indices, replay_i64, weights, indices, indices_i64, prob,
+               zm != 0.f ? zp : nullptr};
+    t.part = base;
+    t.S = g.S;
+    t.ld_p = g.ld_p;
+    t.bias = bias;
+    t.bias_bf16 = w_dtype == FM_DTYPE_BF16;
+    t.score_bias = score_bias;
+    t.logits_out = logits;
+    t.hist = hist;
+    if (int rc = router_gate_launch(t, gb, s, "fm_router_forward")) return rc;
+    hipLaunchKernelGGL(router_finish_wide_kernel, dim3(1), dim3(1024), 0, s, hist, gb, E, counts, tokens_per_expert,
+                       total_tokens, T, prob, zm != 0.f ? zp : nullptr, zm, loss);
+    return check_launch("fm_router_forward");
+  }
+  // fp32 x: logits, then gating, counts and loss as separate kernels
   float* part = base;
   float* zpart = base + kRouterForwardWaves * E;
   if (int rc = router_logits_launch(a, x_dtype, nullptr, 0, s, "fm_router_forward")) return rc;
@@ -1165,7 +1334,9 @@ int fm_gating_grad_dot(const float* logits, int64_t T, int E, int64_t ld_l, int 
 
 int64_t fm_router_workspace_bytes(int64_t T, int64_t D, int E) {
   if (T <= 0 || D <= 0 || E <= 0) return 0;
-  return router_slices(T, D, E) * int64_t(E) * (D + 1) * int64_t(sizeof(float));
+  const int64_t valu = router_slices(T, D, E) * int64_t(E) * (D + 1) * int64_t(sizeof(float));
+  const int64_t mfma = gate_bwd_mfma(D, E) ? gate_bwd_shape(T, D, E).bytes : 0;
+  return valu > mfma ? valu : mfma;
 }
 
 int fm_router_backward(const float* dlogits, int64_t ld_dl, const void* x, int x_dtype, int64_t ld_x, int64_t T,
@@ -1188,6 +1359,11 @@ int fm_router_backward(const float* dlogits, int64_t ld_dl, const void* x, int x
                "fm_router_backward: workspace of fm_router_workspace_bytes(T, D, E) bytes required");
   if (T == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // on the matrix cores (without a workspace only dx can be asked for)
+  if (gate_bwd_mfma(D, E) && x_dtype == FM_DTYPE_BF16 && (dx || dw || db) && aligned16(workspace) && workspace != nullptr &&
+      workspace_bytes >= gate_bwd_shape(T, D, E).bytes)
+    return router_backward_mfma(dlogits, ld_dl, x, ld_x, T, D, w, w_dtype == FM_DTYPE_BF16, ld_w, E, dx, ld_dx, dw,
+                                dw_dtype == FM_DTYPE_BF16, ld_dw, db, db_dtype == FM_DTYPE_BF16, workspace, s);
   RouterBwdArgs a{dlogits, ld_dl, x, ld_x, T, D, w, ld_w, w_dtype == FM_DTYPE_BF16, E, dx, ld_dx,
                   static_cast<float*>(workspace), nullptr, 1, T};
   if (dx != nullptr) {

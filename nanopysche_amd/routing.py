@@ -444,15 +444,13 @@ def router_backward(state: RouterState, x2, gate_weight, dweights, daux, need_x=
     dx = torch.empty_like(x2) if need_x else None
     dW = torch.empty(E, D, dtype=w.dtype, device=dev) if need_w else None
     db = torch.empty(E, dtype=bias_dtype or torch.float32, device=dev) if need_b else None
-    ws = None
-    if dW is not None or db is not None:
-        ws = torch.empty(int(_lib.load().fm_router_workspace_bytes(T, D, E)), dtype=torch.uint8, device=dev)
     if dx is not None or dW is not None or db is not None:
+        ws = torch.empty(int(_lib.load().fm_router_workspace_bytes(T, D, E)), dtype=torch.uint8, device=dev)
         _lib.call("fm_router_backward", _lib.ptr(dlogits), dlogits.stride(0), _lib.ptr(x2), _x_dtype(x2),
                   x2.stride(0), T, D, _lib.ptr(w), _dt_code(w), w.stride(0), E, _lib.ptr(dx),
                   0 if dx is None else dx.stride(0), _lib.ptr(dW), _lib.DTYPE_F32 if dW is None else _dt_code(dW),
                   0 if dW is None else dW.stride(0), _lib.ptr(db), _lib.DTYPE_F32 if db is None else _dt_code(db),
-                  _lib.ptr(ws), 0 if ws is None else ws.numel(), st)
+                  _lib.ptr(ws), ws.numel(), st)
     return dx, dW, db, dlogits
 
 

@@ -1,0 +1,89 @@
+"""The router's products on the matrix cores (bf16 x; fp32 factors as three bf16
+pieces) at the edges of their tiles, against float64: token tiles of 16 / 32 /
+64, expert fragments and groups, chunks of D with a part-filled last step,
+slices of tokens.
+
+Bounds: every product of pieces is exact in fp32, so a sum over n is off by at
+most (n + 2) 2^-24 sum |terms|, the 2 for the low pieces joining the high ones
+(n 2^-23 for the six pairs of pieces of two fp32 factors, which leave out
+terms below 2^-24 of a product)."""
+
+import pytest
+import torch
+
+import nanopysche_amd as fm
+from nanopysche_amd.routing import router_backward, router_forward
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 8, 9), (16, 72, 16), (17, 136, 17), (33, 264, 33), (65, 1000, 48), (130, 512, 64), (200, 776, 65),
+          (64, 2048, 128), (129, 1160, 160), (1000, 384, 256), (37, 200, 5), (100, 4104, 3),
+          (3001, 128, 250)]
+
+
+def _inputs(dev, T, D, E, gate, seed=3):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(T, D, generator=g).bfloat16().to(dev)
+    w = (torch.randn(E, D, generator=g) * 0.05).to(gate).to(dev)
+    b = (torch.randn(E, generator=g) * 0.1).to(gate).to(dev)
+    sb = (torch.randn(E, generator=g) * 0.2).to(dev)
+    return g, x, w, b, sb
+
+
+@pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,D,E", SHAPES)
+def test_products_at_tile_edges(dev, T, D, E, gate):
+    g, x, w, b, sb = _inputs(dev, T, D, E, gate)
+    K = min(E, 6)
+    wts, idx, aux, st = router_forward(x, w, b, sb, K, "softmax", None, None, 1e-3)
+    x64, w64 = x.double(), w.double()
+    ref = x64 @ w64.t() + b.double() + sb.double()
+    bound = (D + 2) * 2.0 ** -24 * (x64.abs() @ w64.abs().t() + b.double().abs() + sb.double().abs()) + 1e-30
+    assert torch.all((st.logits.double() - ref).abs() <= bound)
+    # the selection, counts and loss of these logits
+    lg = st.logits.double()
+    assert torch.equal(torch.gather(lg, 1, idx), lg.topk(K, dim=1).values)
+    assert torch.equal(st.counts.long(), torch.bincount(idx.flatten(), minlength=E))
+    probs = torch.softmax(lg, dim=1)
+    loss = E * (st.counts.double() / T * probs.mean(dim=0)).sum() + 1e-3 * torch.logsumexp(lg, 1).square().mean()
+    assert abs(float(aux) - float(loss)) <= 1e-5 * abs(float(loss))
+    # backward: dx, dw, db of the dlogits it forms
+    dws = torch.randn(T, K, generator=g).to(dev)
+    daux = torch.tensor(0.5, device=dev)
+    dx, dW, db, dl = router_backward(st, x, w, dws, daux, bias_dtype=torch.float32)
+    dl64 = dl.double()
+    size = dl64.abs() @ w64.abs()
+    assert torch.all((dx.double() - dl64 @ w64).abs() <= 2.0 ** -8 * (dl64 @ w64).abs() + (E + 2) * 2.0 ** -23 * size + 1e-30)
+    size = dl64.abs().t() @ x64.abs()
+    out = 2.0 ** -8 if gate == torch.bfloat16 else 0.0
+    assert torch.all((dW.double() - dl64.t() @ x64).abs() <= out * (dl64.t() @ x64).abs() + (T + 2) * 2.0 ** -24 * size + 1e-30)
+    assert torch.all((db.double() - dl64.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * dl64.abs().sum(0) + 1e-30)
+    only = router_backward(st, x, w, dws, daux, need_w=False, need_b=False)[0]
+    assert torch.equal(only, dx)
+
+
+@pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
+def test_infinite_and_nan_inputs(dev, gate):
+    """A non-finite x or gate value reaches the outputs it reaches in fp32 arithmetic, as the same class."""
+    T, D, E = 70, 264, 40
+    _, x, w, b, sb = _inputs(dev, T, D, E, gate)
+    w[3, 5], w[4, 6] = float("inf"), float("nan")
+    x[9, 7], x[10, 8], x[11, 9] = float("inf"), float("-inf"), float("nan")
+    w[:, 9] = 0.25      # a value whose low pieces are zero, against the infinities
+    x[12, 9] = float("inf")
+    got = fm.router_logits(x, w, b, sb)
+    ref = x.float() @ w.float().t() + b.float() + sb
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(ref))
+
+
+def test_selection_order_of_special_scores(dev):
+    """NaN above every number, ties (-0 and +0 among them) to the lower expert, -inf still selectable."""
+    E, K = 200, 5
+    lg = torch.full((4, E), float("-inf"))
+    lg[0, 150], lg[0, 20] = 1.0, 1.0
+    lg[1, 199], lg[1, 64], lg[1, 65] = float("nan"), float("inf"), float("inf")
+    lg[2, 3], lg[2, 70] = -0.0, 0.0
+    lg[3] = 2.0
+    _, idx = fm.topk_gating(lg.to(dev), K)
+    assert idx.cpu().tolist() == [[20, 150, 0, 1, 2], [199, 64, 65, 0, 1], [3, 70, 0, 1, 2], [0, 1, 2, 3, 4]]
