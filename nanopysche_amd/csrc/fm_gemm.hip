@@ -26,16 +26,11 @@
 //              promotion.
 //   FP8_MX     e4m3 with e8m0 scales per 32 (OCP MXFP8), same instruction.
 //
-// Two kernels, K step 128 bytes (128 e4m3 / 64 bf16), operands streamed into
-// LDS by direct global->LDS loads, each wave 128 x 64 = 4 x 2 MFMA 32x32 blocks:
-//   gemm256_kernel  BF16 / FP8_POW2 / FP8_MX.  Tile 256 x 256, 512 threads =
-//                   8 wave64 as 2 (i) x 4 (j), two waves per SIMD, two LDS
-//                   stages of 66 KiB.  In ragged-M a 256-token tile covers two
-//                   128-row groups of one expert; its second half is idle at
-//                   an odd group end.
-//   gemm_f32_kernel FP8_F32.  Tile 256 x 128, 256 threads = 4 wave64 as
-//                   2 x 2, three LDS stages; each 128-deep partial sum is
-//                   promoted through a second set of accumulator registers.
+// One tile, K step 128 bytes (128 e4m3 / 64 bf16), operands streamed into LDS by
+// direct global->LDS loads: 256 x 256, 512 threads = 8 wave64 as 2 (i) x 4 (j),
+// each wave 128 x 64 = 4 x 2 MFMA 32x32 blocks, two waves per SIMD, two LDS
+// stages of 66 KiB.  In ragged-M a 256-token tile covers two 128-row groups of one
+// expert; its second half is idle at an odd group end.
 // Ragged-M workgroup ids are remapped so each XCD walks a contiguous range of
 // the valid tiles, grouped 8 token tiles at a time for L2 reuse of weights and
 // activations; within a group the weight tiles vary fastest when an expert's
@@ -751,6 +746,61 @@ __device__ __forceinline__ bool decode_tile256(const GemmParams& p, Tile256& t, 
   return true;
 }
 
+// FP8_F32: one 128-deep K step of a wave's 128 x 64 block from a stage, each
+// 32 x 32 block's partial sum (both halves of the step, scales neutral) promoted
+// into its accumulators with the product of the two block scales.  The B
+// fragments of both halves stay in registers and the A fragments stream, so
+// accumulators, partial sums and fragments fit 256 registers and two waves
+// share a SIMD: one wave's promotion (16 FMAs a block, and 16 products where
+// both scales differ by row) runs on the VALU beside the other's MFMAs.  Per
+// SIMD and block that is 2 MFMAs (128 cycles) against 17 or 33 VALU
+// instructions (68 or 132).  Measured (8 experts of 750 rows, D 2048, H 1408), against a
+// 256 x 128 tile with one wave per SIMD: gate|up 109 -> 69 us (264 tiles, a second
+// round of 8), down 56 -> 29, dX 104 -> 54, dW1|dW3 181 -> 86.
+template <int MODE>
+__device__ __forceinline__ void f32_step(const uint8_t* st, v16f (&acc)[4][2], const WaveCoord& w) {
+  using SM = Smem256<GK_FP8_F32>;
+  const float* qs = reinterpret_cast<const float*>(st + SM::kQS) + w.wi * 128;
+  const float* ps = reinterpret_cast<const float*>(st + SM::kPS) + w.wj * 64 + w.lrow;
+  const uint8_t* lp = st + SM::kP;
+  v8i fb[2][2];
+  float sp[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) fb[h][b] = read_frag8(lp, w.wj * 64 + b * 32 + w.lrow, h, w.lhalf);
+    sp[b] = ps[b * 32];
+    if (MODE == GM_RAGGED_M) sp[b] = qs[0] * sp[b];   // a wave's 128 weight rows are one scale block
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const v8i fa0 = read_frag8(st, w.wi * 128 + a * 32 + w.lrow, 0, w.lhalf);
+    const v8i fa1 = read_frag8(st, w.wi * 128 + a * 32 + w.lrow, 1, w.lhalf);
+    float4 sq[4];
+    if (MODE == GM_RAGGED_K)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) sq[g] = *reinterpret_cast<const float4*>(qs + a * 32 + 8 * g + 4 * w.lhalf);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      v16f part;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[r] = 0.f;
+      part = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa0, fb[0][b], part, 0, 0, 0, 127, 0, 127);
+      part = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa1, fb[1][b], part, 0, 0, 0, 127, 0, 127);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if (MODE == GM_RAGGED_M) {
+          acc[a][b][r] += part[r] * sp[b];
+        } else {
+          const float4 v = sq[r >> 2];
+          const float q = (r & 3) == 0 ? v.x : (r & 3) == 1 ? v.y : (r & 3) == 2 ? v.z : v.w;
+          acc[a][b][r] += part[r] * (q * sp[b]);
+        }
+      }
+    }
+  }
+}
+
 // One 256 x 256 output tile of launch `p` (block index `bid` of that launch,
 // two LDS stages at `smem`).  MXL (MX only): scale layouts, bit 0 = Q scales
 // k-major, bit 1 = P scales k-major (row-major otherwise); fixed per
@@ -813,7 +863,22 @@ __device__ __forceinline__ void gemm256_tile(const GemmParams& p, int64_t bid, u
   // are unconditional (clamped to the last step), which keeps the loop body
   // one basic block; the reads after the last step re-read a valid stage.
   const int64_t nk = (k_hi - k_lo) / KSTEP;
-  if (nk > 0) {
+  if constexpr (KIND == GK_FP8_F32) {
+    // one barrier a step: stage t % 2 has landed for every wave and no wave still
+    // reads the other, which takes step t + 1 while this one is computed
+    const uint32_t smem_lds = lds_addr(smem);
+    if (nk > 0) issue_step<KIND>(qst, pst, sc, k_lo, smem_lds, w.wave);
+    int cur_off = 0;
+#pragma unroll 1
+    for (int64_t t = 0; t < nk; ++t) {
+      FM_WAIT_VMCNT(0);
+      block_barrier();
+      const int nxt_off = SM::kStage - cur_off;
+      if (t + 1 < nk) issue_step<KIND>(qst, pst, sc, k_lo + (t + 1) * KSTEP, smem_lds + nxt_off, w.wave);
+      f32_step<MODE>(smem + cur_off, acc, w);
+      cur_off = nxt_off;
+    }
+  } else if (nk > 0) {
     const uint32_t smem_lds = lds_addr(smem);
     Frag<KIND> f0, f1;
     issue_step<KIND>(qst, pst, sc, k_lo, smem_lds, w.wave);
@@ -2260,268 +2325,6 @@ __global__ __launch_bounds__(512) void gemm256r_kernel(GemmParams pm, GemmParams
 }
 
 // ============================================================================
-// 256 x 128 kernel: FP8_F32 (fp32 block scales, promotion per 128-deep block)
-// ============================================================================
-constexpr int kBI = 256;   // workgroup tile along i (weight rows / M)
-constexpr int kBJ = 128;   // workgroup tile along j (tokens / N)
-
-struct SmemF32 {
-  static constexpr int kQ = kBI * 128;                 // operand bytes per stage
-  static constexpr int kP = kBJ * 128;
-  static constexpr int kQS = kBI * 4;                  // scale bytes per stage
-  static constexpr int kPS = kBI * 4;                  // 256 slots, the upper 128 unused
-  static constexpr int kStage = kQ + kP + kQS + kPS;
-};
-
-// Per-lane DMA sources of one workgroup tile.
-struct TileSrc {
-  const uint8_t* q[8];   // 8 x 1 KiB of the 256-row operand per wave
-  const uint8_t* p[4];   // 4 x 1 KiB of the 128-row operand per wave
-  const uint8_t* qs;     // scale word of this lane (Q side)
-  const uint8_t* ps;     // scale word of this lane (P side; rows past 128 re-read row 127)
-  int64_t qs_k, ps_k;    // scale byte advance per K step
-};
-
-__device__ __forceinline__ void f32_issue(const TileSrc& src, int64_t k, uint8_t* stage, int wave) {
-  using SM = SmemF32;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) dma16(src.q[u] + k, stage + (wave * 8 + u) * 1024);
-#pragma unroll
-  for (int u = 0; u < 4; ++u) dma16(src.p[u] + k, stage + SM::kQ + (wave * 4 + u) * 1024);
-  const int64_t ks = k / 128;
-  dma4(src.qs + ks * src.qs_k, stage + SM::kQ + SM::kP + wave * 256);
-  dma4(src.ps + ks * src.ps_k, stage + SM::kQ + SM::kP + SM::kQS + wave * 256);
-}
-
-// One 128-deep K step from a stage: 4 x 2 MFMA 32x32 blocks per wave, each
-// 128-deep partial sum promoted with the product of the block scales.
-template <int MODE>
-__device__ __forceinline__ void f32_compute(const uint8_t* st, v16f (&acc)[4][2], int wi, int wj,
-                                            int lrow, int lhalf) {
-  using SM = SmemF32;
-  const uint8_t* lq = st;
-  const uint8_t* lp = st + SM::kQ;
-  const float* qs = reinterpret_cast<const float*>(st + SM::kQ + SM::kP);
-  const float* ps = reinterpret_cast<const float*>(st + SM::kQ + SM::kP + SM::kQS);
-  v8i fa[2][4], fb[2][2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) fa[ks][t] = read_frag8(lq, wi * 128 + t * 32 + lrow, ks, lhalf);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) fb[ks][t] = read_frag8(lp, wj * 64 + t * 32 + lrow, ks, lhalf);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      v16f part;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) part[r] = 0.f;
-      part = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[0][a], fb[0][b], part, 0, 0, 0, 127, 0, 127);
-      part = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[1][a], fb[1][b], part, 0, 0, 0, 127, 0, 127);
-      const float sp = ps[wj * 64 + b * 32 + lrow];
-      if (MODE == GM_RAGGED_M) {
-        const float s = qs[wi * 128] * sp;  // a wave's 128 rows are one 128x128 weight block
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] += part[r] * s;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int ii = wi * 128 + a * 32 + 8 * (r >> 2) + 4 * lhalf + (r & 3);
-          acc[a][b][r] += part[r] * (qs[ii] * sp);
-        }
-      }
-    }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
-  using SM = SmemF32;
-  constexpr int NLOAD = 14;   // DMA instructions per wave per step
-  // three pipeline stages of one K step each (operands + scales)
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[3 * SM::kStage];
-  uint8_t* const smem0 = smem;
-  uint8_t* const smem1 = smem + SM::kStage;
-  uint8_t* const smem2 = smem + 2 * SM::kStage;
-
-  // ---------------------------------------------------------- tile decode ----
-  // ragged-M: the valid 128-row tiles [0, offsets[E] / 128) split into one
-  // contiguous range per XCD; ragged-K: tiles in launch order (as above).
-  int64_t e = -1, i0 = 0, j0 = 0, k_lo, k_hi;
-  const int64_t NI = (p.n_i + kBI - 1) / kBI;
-  int64_t L;
-  // 128-row tiles of unmasked experts only (see the 256-tile kernel)
-  auto unmasked = [&](int x) { return p.mask == nullptr || p.mask[x] == p.mask_want; };
-  int64_t MT = 0;
-  if (MODE == GM_RAGGED_M) {
-    for (int x = 0; x < p.E; ++x)
-      if (unmasked(x)) MT += (p.offsets[x + 1] - p.offsets[x]) / kBJ;
-    const int64_t n_valid = MT * NI;
-    const int64_t per_xcd = (n_valid + 7) / 8;
-    const int64_t k = blockIdx.x / 8;
-    if (k >= per_xcd) return;
-    L = int64_t(blockIdx.x % 8) * per_xcd + k;
-    if (L >= n_valid) return;
-  } else {
-    L = blockIdx.x;
-    if (L >= p.n_tiles) return;
-  }
-  if (MODE == GM_RAGGED_M) {
-    const int64_t group = L / (kGroupM * NI);
-    const int64_t first = group * kGroupM;
-    const int64_t gsz = MT - first < kGroupM ? MT - first : kGroupM;
-    int64_t mt = first + (L % gsz);
-    const int64_t nt = (L % (kGroupM * NI)) / gsz;
-    for (int x = 0; x < p.E; ++x) {
-      const int64_t o0 = p.offsets[x];
-      const int64_t cnt = unmasked(x) ? (p.offsets[x + 1] - o0) / kBJ : 0;
-      if (mt < cnt) {
-        e = x;
-        j0 = o0 + mt * kBJ;
-        break;
-      }
-      mt -= cnt;
-    }
-    if (e < 0) return;
-    i0 = nt * kBI;
-    k_lo = 0;
-    k_hi = p.K;
-  } else {
-    const int64_t NJ = p.n_j / kBJ;
-    const int64_t per_e = NI * NJ;
-    e = L / per_e;
-    const int64_t Lr = L % per_e;
-    const int64_t group = Lr / (kGroupM * NJ);
-    const int64_t first = group * kGroupM;
-    const int64_t gsz = NI - first < kGroupM ? NI - first : kGroupM;
-    i0 = (first + (Lr % gsz)) * kBI;
-    j0 = ((Lr % (kGroupM * NJ)) / gsz) * kBJ;
-    k_lo = p.offsets[e];
-    k_hi = p.offsets[e + 1];
-  }
-  if (p.mask != nullptr && p.mask[e] != p.mask_want) return;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wi = wave >> 1, wj = wave & 1;   // wave tile: i [128*wi, +128), j [64*wj, +64)
-  const int lrow = lane & 31, lhalf = lane >> 5;
-  const int64_t q_group = MODE == GM_RAGGED_M ? e : 0;
-  const int64_t i_last = p.n_i - 1;
-
-  // ------------------------------------------------ per-lane DMA sources ----
-  // Linear LDS chunk c = 64*instr + lane of a tile of 128-byte rows holds row
-  // c/8, swizzled chunk (c%8) ^ lds_swz(row); each lane fetches the global 16
-  // bytes that belong there.  Rows past the end of Q (an N tail) re-read the last row.
-  TileSrc src;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int c = (wave * 8 + u) * 64 + lane;
-    const int row = c >> 3, ch = (c & 7) ^ lds_swz(row);
-    int64_t gr = i0 + row;
-    gr = gr < i_last ? gr : i_last;
-    src.q[u] = p.Q.p + (q_group * p.Q.gs + gr * p.Q.ld) + ch * 16;
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = (wave * 4 + u) * 64 + lane;
-    const int row = c >> 3, ch = (c & 7) ^ lds_swz(row);
-    src.p[u] = p.P.p + ((j0 + row) * p.P.ld) + ch * 16;
-  }
-  // Scales: one row per lane, Q 256 rows, P 128 rows (lanes for P rows 128-255
-  // re-read row 127 into unused slots, so every wave issues the same loads).
-  {
-    const int qi = wave * 64 + lane;
-    int64_t gr = i0 + qi;
-    gr = gr < i_last ? gr : i_last;
-    src.qs = static_cast<const uint8_t*>(p.Q.s) + (q_group * p.Q.s_gs + (gr >> p.Q.s_shift) * p.Q.s_row) * 4;
-    const int pc = qi < kBJ ? qi : kBJ - 1;
-    src.ps = static_cast<const uint8_t*>(p.P.s) + ((j0 + pc) >> p.P.s_shift) * p.P.s_row * 4;
-    src.qs_k = p.Q.s_kb * 4;
-    src.ps_k = p.P.s_kb * 4;
-  }
-
-  v16f acc[4][2];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
-  // Pipeline: stage t % 3 is filled two steps ahead.  Readiness of a stage is
-  // this wave's own vmcnt wait (DMA writes land in LDS before the counter
-  // drops) followed by a barrier; a stage is refilled only after every wave has
-  // passed the barrier that follows its last read of it.
-  const int64_t nk = (k_hi - k_lo) / 128;
-  if (nk > 0) f32_issue(src, k_lo, smem0, wave);
-  if (nk > 1) f32_issue(src, k_lo + 128, smem1, wave);
-  // Main loop: steps with a successor, whose loads are always in flight here,
-  // so an unconditional vmcnt(NLOAD) retires exactly the current stage's DMA.
-  int64_t t = 0;
-  while (t + 1 < nk) {
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      if (t + 1 >= nk) break;
-      FM_WAIT_VMCNT(NLOAD);
-      block_barrier();
-      uint8_t* nxt = u == 0 ? smem2 : (u == 1 ? smem0 : smem1);
-      const uint8_t* cur = u == 0 ? smem0 : (u == 1 ? smem1 : smem2);
-      // unconditional: at t = nk-2 this re-reads step nk-1 into the stage of
-      // step nk, which is never read
-      const int64_t tn = t + 2 < nk ? t + 2 : nk - 1;
-      f32_issue(src, k_lo + tn * 128, nxt, wave);
-      f32_compute<MODE>(cur, acc, wi, wj, lrow, lhalf);
-      ++t;
-    }
-  }
-  if (t < nk) {  // last step: nothing else in flight
-    FM_WAIT_VMCNT(0);
-    block_barrier();
-    const int sidx = int(t % 3);
-    const uint8_t* cur = sidx == 0 ? smem0 : (sidx == 1 ? smem1 : smem2);
-    f32_compute<MODE>(cur, acc, wi, wj, lrow, lhalf);
-  }
-
-  // -------------------------------------------------------------- epilogue ----
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int64_t j = j0 + wj * 64 + b * 32 + lrow;
-      if (MODE == GM_RAGGED_M) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int64_t i = i0 + wi * 128 + a * 32 + 8 * q + 4 * lhalf;
-          if (i >= p.n_i) continue;
-          if (p.out_f32) {
-            float* dst = static_cast<float*>(p.C) + j * p.ldC + i;
-            st_global(dst,
-                make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]));
-          } else {
-            uint16_t* dst = static_cast<uint16_t*>(p.C) + j * p.ldC + i;
-            uint2 v;
-            v.x = hw_bf16x2(acc[a][b][4 * q], acc[a][b][4 * q + 1]);
-            v.y = hw_bf16x2(acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
-            st_global(dst, v);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t i = i0 + wi * 128 + a * 32 + 8 * (r >> 2) + 4 * lhalf + (r & 3);
-          if (i >= p.n_i) continue;
-          const bool second = i >= p.split;
-          const int64_t row = second ? i - p.split : i;
-          const int64_t off = e * (second ? p.c2_gs : p.c_gs) + row * p.ldC + j;
-          void* base = second ? p.C2 : p.C;
-          if (p.out_f32) st_global(static_cast<float*>(base) + off, acc[a][b][r]);
-          else st_global(static_cast<uint16_t*>(base) + off, f32_to_bf16(acc[a][b][r]));
-        }
-      }
-    }
-}
-
-// ============================================================================
 // launch
 // ============================================================================
 // FM_RK_XCD=0: ragged-K launches keep their tiles in launch order even for
@@ -2659,6 +2462,7 @@ inline void launch256(int kind, dim3 grid, const GemmParams& p, hipStream_t s) {
   const dim3 block(512);
   switch (kind) {
     case GK_BF16: hipLaunchKernelGGL((gemm256_kernel<GK_BF16, MODE>), grid, block, 0, s, p); break;
+    case GK_FP8_F32: hipLaunchKernelGGL((gemm256_kernel<GK_FP8_F32, MODE>), grid, block, 0, s, p); break;
     case GK_FP8_POW2: hipLaunchKernelGGL((gemm256_kernel<GK_FP8_POW2, MODE>), grid, block, 0, s, p); break;
     default: {
       const int mxl = (p.Q.s_kb != 1 ? 1 : 0) | (p.P.s_kb != 1 ? 2 : 0);
@@ -2679,7 +2483,7 @@ int prepare_gemm(int kind, GemmParams& p) {
     set_error("grouped gemm: unknown kind %d", kind);
     return 1;
   }
-  if (MODE == GM_RAGGED_K && kind != GK_FP8_F32) {
+  if (MODE == GM_RAGGED_K) {
     // the 256 x 256 kernel writes rows along j: put the output's row operand
     // (a_t, M rows) on the P side and its column operand (b_t) on the Q side
     const Operand t = p.P;
@@ -2690,14 +2494,9 @@ int prepare_gemm(int kind, GemmParams& p) {
     p.n_j = n;
   }
   const int64_t NI256 = (p.n_i + kT - 1) / kT;
-  if (kind == GK_FP8_F32) {
-    const int64_t NI = (p.n_i + kBI - 1) / kBI;
-    p.n_tiles = MODE == GM_RAGGED_M ? p.m_tiles * NI : int64_t(p.E) * NI * (p.n_j / kBJ);
-  } else {
-    if (p.splits < 1) p.splits = 1;
-    p.n_tiles = MODE == GM_RAGGED_M ? p.j_tiles * NI256
-                                    : int64_t(p.E) * NI256 * ((p.n_j + kT - 1) / kT) * p.splits;
-  }
+  if (p.splits < 1) p.splits = 1;
+  p.n_tiles = MODE == GM_RAGGED_M ? p.j_tiles * NI256
+                                  : int64_t(p.E) * NI256 * ((p.n_j + kT - 1) / kT) * p.splits;
   p.rk_xcd = MODE == GM_RAGGED_K ? (gemm_rk_xcd_split() ? 1 : 0) | (gemm_rk_chunked() ? 2 : 0) : 0;
   p.w_fast = MODE == GM_RAGGED_M && gemm_weight_fast(p.n_i * p.K * (kind == GK_BF16 ? 2 : 1)) ? 1 : 0;
   return 0;
@@ -2707,9 +2506,9 @@ template <int MODE>
 int dispatch_gemm(int kind, GemmParams p, hipStream_t s) {
   if (int rc = prepare_gemm<MODE>(kind, p)) return rc;
   if (p.n_tiles == 0) return 0;
-  const dim3 grid(unsigned((p.n_tiles + 7) / 8 * 8)), block(256);
+  const dim3 grid(unsigned((p.n_tiles + 7) / 8 * 8));
   if (kind == GK_FP8_F32) {
-    hipLaunchKernelGGL((gemm_f32_kernel<MODE>), grid, block, 0, s, p);
+    launch256<MODE>(kind, grid, p, s);
   } else if (MODE == GM_RAGGED_M && p.E <= 64 && p.K / (kind == GK_BF16 ? 64 : 128) >= 2 &&
              (gemm_persistent() || p.q_nn || p.paired || p.Q.split != INT64_MAX)) {
     launch256p(kind, p, s);
