@@ -8,6 +8,7 @@ device is present when a kernel is requested, the call raises.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import threading
 from pathlib import Path
 
@@ -189,8 +190,22 @@ def check(rc: int, what: str = "") -> None:
         raise RuntimeError(f"libfm_hip {what} failed (code {rc}): {msg}")
 
 
+_fns = {}
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc:
+        check(rc, name)
+
+
+@functools.lru_cache(maxsize=4096)
+def size_of(name: str, *args: int) -> int:
+    """A size function of the library (pure in its arguments)."""
+    return int(getattr(load(), name)(*args))
 
 
 def require_device(t: torch.Tensor, name: str = "tensor") -> None:
@@ -200,9 +215,16 @@ def require_device(t: torch.Tensor, name: str = "tensor") -> None:
             "(there is no CPU fallback)")
 
 
-def stream_of(t: torch.Tensor) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def stream_of(t: torch.Tensor) -> int:
+    """The handle of the current stream of t's device (0.1 us; through a
+    torch.cuda.Stream object it took 2.2 us, once per launch)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t) -> C.c_void_p:
     return C.c_void_p(0 if t is None else t.data_ptr())
+
+
+def addr(t):
+    """ptr as the plain integer (or None) that ctypes converts itself."""
+    return None if t is None else t.data_ptr()

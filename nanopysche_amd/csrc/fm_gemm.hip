@@ -75,7 +75,7 @@ struct GemmParams {
   int64_t n_i;        // extent of i (rows of Q per group)
   int64_t n_j;        // ragged-K: extent of j (rows of P)
   int64_t K;          // ragged-M: contraction length
-  const int32_t* tile_expert;  // ragged-M, 256 x 128 kernel: expert of each 128-row tile
+  const int32_t* tile_expert;  // ragged-M: expert of each 128-row tile
   int64_t m_tiles;             // ragged-M: 128-row tiles in the padded buffer
   int64_t j_tiles;             // ragged-M, 256 x 256 kernel: bound on 256-row token tiles
   const int32_t* offsets;      // [E+1] padded group starts (rows)
@@ -2823,7 +2823,7 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
     else hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_POW2, 0, true, true, false, true>), pgrid, pblock, 0, s, pm, pk);
     return check_launch("fm_grouped_gemm_ragged_m_k");
   }
-  if (nn || pm.m_tiles == 0 || (kind != GK_BF16 && kind != GK_FP8_POW2) || !gemm_mk_one_grid()) {
+  if (nn || pm.m_tiles == 0 || kind == GK_FP8_MX || !gemm_mk_one_grid()) {
     if (pm.m_tiles > 0)
       if (int rc = dispatch_gemm<GM_RAGGED_M>(kind, pm, s)) return rc;
     return dispatch_gemm<GM_RAGGED_K>(kind, pk, s);
@@ -2833,7 +2833,7 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
   if (int rc = prepare_gemm<GM_RAGGED_K>(kind, pk)) return rc;
   const int64_t nbm = (pm.n_tiles + 7) / 8 * 8, nbk = (pk.n_tiles + 7) / 8 * 8;
   if (nbm + nbk == 0) return 0;
-  if (expert_mask == nullptr && E <= 64 && pm.K / (kind == GK_BF16 ? 64 : 128) >= 2 &&
+  if (kind != GK_FP8_F32 && expert_mask == nullptr && E <= 64 && pm.K / (kind == GK_BF16 ? 64 : 128) >= 2 &&
       pk.n_tiles < (int64_t(1) << 28) && gemm_persistent_k()) {
     // persistent: one workgroup per CU (a multiple of 8), at most one per tile
     const int64_t slots = int64_t(device_cus() / 8 > 0 ? device_cus() / 8 : 1) * 8;
@@ -2848,6 +2848,7 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
   }
   const dim3 grid(unsigned(nbm + nbk)), block(512);
   if (kind == GK_BF16) hipLaunchKernelGGL((gemm256_mk_kernel<GK_BF16>), grid, block, 0, s, pm, pk, nbm);
+  else if (kind == GK_FP8_F32) hipLaunchKernelGGL((gemm256_mk_kernel<GK_FP8_F32>), grid, block, 0, s, pm, pk, nbm);
   else hipLaunchKernelGGL((gemm256_mk_kernel<GK_FP8_POW2>), grid, block, 0, s, pm, pk, nbm);
   return check_launch("fm_grouped_gemm_ragged_m_k");
 }

@@ -118,7 +118,8 @@ def _tile_args(kind, q, s, qt, st, paired=False, col_paired=False):
         kind |= _lib.ROWS_PAIRED
     if col_paired:
         kind |= _lib.COLS_PAIRED
-    return (kind, _lib.ptr(q), _ld(q), _lib.ptr(s), ld_s, _lib.ptr(qt), _ld(qt), _lib.ptr(st), _ld(st))
+    addr = _lib.addr
+    return (kind, addr(q), _ld(q), addr(s), ld_s, addr(qt), _ld(qt), addr(st), _ld(st))
 
 
 def _wrap(q, s, qt, st, kind, paired=False, col_paired=False):
@@ -230,6 +231,53 @@ def scaling_aware_transpose(t: FP8Tensor) -> FP8Tensor:
 
 
 # ======================================================================= SwiGLU ====
+class _Act:
+    """An activation operand inside the expert block: payload, then (from byte
+    ``scale_off`` of one allocation) its scales, as a producer wrote them, with the
+    strides the grouped GEMM reads them by (rows: block-major scales [blocks,
+    rows]; columns: [rows / block, C])."""
+
+    __slots__ = ("buf", "ld", "scale_off", "s_kb", "paired")
+
+    def __init__(self, buf, ld, scale_off, s_kb, paired):
+        self.buf, self.ld, self.scale_off, self.s_kb, self.paired = buf, ld, scale_off, s_kb, paired
+
+
+_ACT_BLOCK = {_lib.QUANT_BLOCK: (FP8_BLOCK_SIZE, 4), _lib.QUANT_POW2: (FP8_BLOCK_SIZE, 4),
+              _lib.QUANT_MX: (MX_BLOCK_SIZE, 1)}
+
+
+def _alloc_act(rows, cols, kind, col, dev, paired, col_paired):
+    """Buffers of a producer inside the expert block (rows and cols multiples of 128):
+    (row _Act, column _Act or None, the producer's kind .. ld_st arguments)."""
+    n = rows * cols
+    if kind == _lib.QUANT_BF16:
+        q = torch.empty(n, dtype=torch.bfloat16, device=dev)
+        qt = torch.empty(n, dtype=torch.bfloat16, device=dev) if col else None
+        return (_Act(q, cols, None, 0, False), _Act(qt, rows, None, 0, False) if col else None,
+                (kind, q.data_ptr(), cols, None, 0, _lib.addr(qt), rows if col else 0, None, 0))
+    blk, size = _ACT_BLOCK[kind]
+    total = n + n // blk * size
+    q = torch.empty(total, dtype=torch.uint8, device=dev)
+    row, at = _Act(q, cols, n, rows, paired), q.data_ptr()
+    code = kind | _lib.SCALES_KMAJOR | (_lib.ROWS_PAIRED if paired else 0)
+    if not col:
+        return row, None, (code, at, cols, at + n, rows, None, 0, None, 0)
+    qt = torch.empty(total, dtype=torch.uint8, device=dev)
+    at_t = qt.data_ptr()
+    return (row, _Act(qt, rows, n, cols, col_paired),
+            (code | (_lib.COLS_PAIRED if col_paired else 0), at, cols, at + n, rows, at_t, rows, at_t + n, cols))
+
+
+def _permute_act(x, plan, kind, col, weights, tile_valid, paired, col_paired):
+    """fused_permute_pad inside the expert block: x [T, D] contiguous bf16, weights [T * K] contiguous fp32 or None."""
+    T, D = x.shape
+    row, c, args = _alloc_act(plan.rows_max, D, kind, col, x.device, paired, col_paired)
+    _lib.call("fm_permute", x.data_ptr(), T, D, D, plan.assign_of_row.data_ptr(), plan.rows_max, plan.top_k,
+              _lib.addr(weights), *args, _lib.ptr(tile_valid), _lib.stream_of(x))
+    return row, c
+
+
 def _swiglu(g, u, rows, H, kind, row, col, dev, tile_valid=None, kmajor=False, paired=False, col_paired=False):
     q, s, qt, st = _alloc_quant(rows, H, kind, row, col, dev, kmajor)
     _lib.call("fm_swiglu_quantize", _lib.ptr(g), g.stride(0), _lib.ptr(u), u.stride(0), rows, H,
@@ -359,12 +407,12 @@ def fused_unpermute_unpad(y: torch.Tensor, plan: RoutingPlan,
         gw = gw.detach()
         if gw.dtype not in (torch.float32, torch.bfloat16) or gw.stride(1) != 1:
             gw = gw.float().contiguous()
-        _lib.call("fm_unpermute_router", _lib.ptr(y), y.stride(0), _lib.ptr(plan.row_of), _lib.ptr(w), T, K, D,
-                  _lib.ptr(out), od, out.stride(0), _lib.ptr(addend), 0 if addend is None else addend.stride(0),
-                  _lib.ptr(dl), dl.stride(0), _lib.ptr(gw), _dt(gw), gw.stride(0), gw.shape[0], _lib.stream_of(y))
+        _lib.call("fm_unpermute_router", _lib.addr(y), y.stride(0), _lib.addr(plan.row_of), _lib.addr(w), T, K, D,
+                  _lib.addr(out), od, out.stride(0), _lib.addr(addend), 0 if addend is None else addend.stride(0),
+                  _lib.addr(dl), dl.stride(0), _lib.addr(gw), _dt(gw), gw.stride(0), gw.shape[0], _lib.stream_of(y))
         return out
-    _lib.call("fm_unpermute", _lib.ptr(y), y.stride(0), _lib.ptr(plan.row_of), _lib.ptr(w), T, K, D,
-              _lib.ptr(out), od, out.stride(0), _lib.ptr(addend), 0 if addend is None else addend.stride(0),
+    _lib.call("fm_unpermute", _lib.addr(y), y.stride(0), _lib.addr(plan.row_of), _lib.addr(w), T, K, D,
+              _lib.addr(out), od, out.stride(0), _lib.addr(addend), 0 if addend is None else addend.stride(0),
               _lib.stream_of(y))
     return out
 
@@ -385,8 +433,21 @@ def _operand(data, scale=None, *, ld=None, gs=0, s_row=0, s_kb=0, s_gs=0, shift=
     return o
 
 
+def _act_operand(t):
+    o = _lib.FmGemmOperand()   # zeros
+    o.data = at = t.buf.data_ptr()
+    o.ld = t.ld
+    if t.scale_off is not None:
+        o.scale = at + t.scale_off
+        o.scale_row_stride = 1
+        o.scale_kb_stride = t.s_kb
+    return o
+
+
 def _token_operand(t, kind):
-    """Row-major activations [rows, K] (FP8Tensor or bf16 tensor)."""
+    """Row-major activations [rows, K] (_Act, FP8Tensor or bf16 tensor)."""
+    if type(t) is _Act:
+        return _act_operand(t)
     if kind == _lib.QUANT_BF16:
         return _operand(t)
     return _operand(t.data, t.scale, s_row=t.scale.stride(0), s_kb=t.scale.stride(1))
@@ -394,6 +455,8 @@ def _token_operand(t, kind):
 
 def _col_operand(t, kind):
     """Column-quantised transposed activations [C, rows] with scales [rows/blk, C]."""
+    if type(t) is _Act:
+        return _act_operand(t)
     if kind == _lib.QUANT_BF16:
         return _operand(t)
     return _operand(t.data, t.scale, s_row=1, s_kb=t.scale.stride(0))
@@ -467,11 +530,14 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
         elif w.paired:
             raise ValueError("paired-row weights need paired-row tokens")
         _lib.call("fm_grouped_gemm_ragged_m", gk, _token_operand(tokens, kind),
-                  w.operand(), plan.m_tiles, _lib.ptr(plan.tile_expert), _lib.ptr(plan.offsets),
+                  w.operand(), plan.m_tiles, _lib.addr(plan.tile_expert), _lib.addr(plan.offsets),
                   plan.num_experts, w.N, w.K,
-                  _lib.ptr(mask), want, _lib.ptr(out), _dt(out), out.stride(0), _lib.stream_of(out))
+                  _lib.addr(mask), want, _lib.addr(out), _dt(out), out.stride(0), _lib.stream_of(out))
 
-    _timed(f"grouped_gemm_ragged_m/{_KIND_NAME[kind]}", 2.0 * _assignments(plan, mask, want) * w.N * w.K, launch)
+    if GEMM_TIMER is None:
+        launch()
+    else:
+        _timed(f"grouped_gemm_ragged_m/{_KIND_NAME[kind]}", 2.0 * _assignments(plan, mask, want) * w.N * w.K, launch)
 
 
 # Model of a ragged-K launch for choosing its K split: ~1.3 us per 128-deep K
@@ -531,28 +597,31 @@ def _gemm_k(kind, a_t, b_t, plan: RoutingPlan, M, N, out, out_gs, out2=None, out
         gk |= _lib.GEMM_PAIRED
     ws = None
     if S > 1:
-        nbytes = int(_lib.load().fm_grouped_gemm_ragged_k_split_workspace_bytes(plan.num_experts, M, N, S))
+        nbytes = _lib.size_of("fm_grouped_gemm_ragged_k_split_workspace_bytes", plan.num_experts, M, N, S)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=out.device)
 
     def launch():
         if ws is None:
             _lib.call("fm_grouped_gemm_ragged_k", gk, _col_operand(a_t, kind),
-                      _col_operand(b_t, kind), _lib.ptr(plan.offsets), plan.num_experts, M, N,
-                      _lib.ptr(mask), want, _lib.ptr(out), out_gs, _lib.ptr(out2), out2_gs,
+                      _col_operand(b_t, kind), _lib.addr(plan.offsets), plan.num_experts, M, N,
+                      _lib.addr(mask), want, _lib.addr(out), out_gs, _lib.addr(out2), out2_gs,
                       M if split is None else split, _dt(out), N, _lib.stream_of(out))
         else:
             _lib.call("fm_grouped_gemm_ragged_k_split", gk, _col_operand(a_t, kind),
-                      _col_operand(b_t, kind), _lib.ptr(plan.offsets), plan.num_experts, M, N,
-                      _lib.ptr(mask), want, _lib.ptr(out), out_gs, _lib.ptr(out2), out2_gs,
-                      M if split is None else split, _dt(out), N, S, _lib.ptr(ws), ws.numel() * 4,
+                      _col_operand(b_t, kind), _lib.addr(plan.offsets), plan.num_experts, M, N,
+                      _lib.addr(mask), want, _lib.addr(out), out_gs, _lib.addr(out2), out2_gs,
+                      M if split is None else split, _dt(out), N, S, _lib.addr(ws), ws.numel() * 4,
                       _lib.stream_of(out))
 
-    _timed(f"grouped_gemm_ragged_k/{_KIND_NAME[kind]}", 2.0 * _assignments(plan, mask, want) * M * N, launch)
+    if GEMM_TIMER is None:
+        launch()
+    else:
+        _timed(f"grouped_gemm_ragged_k/{_KIND_NAME[kind]}", 2.0 * _assignments(plan, mask, want) * M * N, launch)
 
 
 # Kinds whose dgrad and weight-gradient launches can share one grid
-# (fm_grouped_gemm_ragged_m_k); the others run them on two streams.
-_MK_KINDS = (_lib.QUANT_BF16, _lib.QUANT_POW2)
+# (fm_grouped_gemm_ragged_m_k); MX runs them on two streams.
+_MK_KINDS = (_lib.QUANT_BF16, _lib.QUANT_POW2, _lib.QUANT_BLOCK)
 
 
 def _gemm_mk(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, a_t, b_t, M2, N2, out2, out2_gs,
@@ -569,13 +638,16 @@ def _gemm_mk(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, a_t, 
 
     def launch():
         _lib.call("fm_grouped_gemm_ragged_m_k", gk, _token_operand(tokens, kind), w.operand(), plan.m_tiles,
-                  _lib.ptr(plan.tile_expert), w.N, w.K, _lib.ptr(out), _dt(out), out.stride(0),
-                  _col_operand(a_t, kind), _col_operand(b_t, kind), M2, N2, _lib.ptr(out2), out2_gs, None, 0, M2,
-                  _dt(out2), N2, _lib.ptr(plan.offsets), plan.num_experts, _lib.ptr(mask), want,
+                  _lib.addr(plan.tile_expert), w.N, w.K, _lib.addr(out), _dt(out), out.stride(0),
+                  _col_operand(a_t, kind), _col_operand(b_t, kind), M2, N2, _lib.addr(out2), out2_gs, None, 0, M2,
+                  _dt(out2), N2, _lib.addr(plan.offsets), plan.num_experts, _lib.addr(mask), want,
                   _lib.stream_of(out))
 
-    _timed(f"grouped_gemm_ragged_m_k/{_KIND_NAME[kind]}",
-           2.0 * _assignments(plan, mask, want) * (w.N * w.K + M2 * N2), launch)
+    if GEMM_TIMER is None:
+        launch()
+    else:
+        _timed(f"grouped_gemm_ragged_m_k/{_KIND_NAME[kind]}",
+               2.0 * _assignments(plan, mask, want) * (w.N * w.K + M2 * N2), launch)
 
 
 def _dt(t):
@@ -676,7 +748,7 @@ class ExpertWeights:
         the buffers, which every replay rewrites, are not kept as the cache of
         later eager calls."""
         key = tuple((w.data_ptr(), w._version, w.dtype) for w in (w1, w2, w3))
-        capturing = torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+        capturing = _capturing()
         if capturing or key != self.key or (need_dgrad and not self.has_dgrad):
             self.key = None
             self.w13 = self.w2t = self.w2 = self.w13t = None
@@ -735,10 +807,10 @@ class ExpertWeights:
 
         def job(src, dst, s, dst_t, s_t, row_off, col_off, rows_out):
             return _lib.FmWeightJob(
-                _lib.ptr(src), _src_dtype(src), E, H, D, D, H * D, kind,
-                _lib.ptr(dst), D, rows_out * D, row_off, _lib.ptr(s), D // 128, (rows_out // 128) * (D // 128),
-                _lib.ptr(dst_t), rows_out, D * rows_out, col_off,
-                _lib.ptr(s_t), rows_out // 128, (D // 128) * (rows_out // 128))
+                _lib.addr(src), _src_dtype(src), E, H, D, D, H * D, kind,
+                _lib.addr(dst), D, rows_out * D, row_off, _lib.addr(s), D // 128, (rows_out // 128) * (D // 128),
+                _lib.addr(dst_t), rows_out, D * rows_out, col_off,
+                _lib.addr(s_t), rows_out // 128, (D // 128) * (rows_out // 128))
 
         # w1 and w3 into the rows (and transposed columns) of the [E, 2H, D] gate|up
         # operand, w2 into its transpose (and its own rows): one launch
@@ -771,8 +843,8 @@ class ExpertWeights:
 
         def job(src, dst, s, row_off, rows_out, pair=False):
             return _lib.FmWeightJob(
-                _lib.ptr(src), _src_dtype(src), E, H, D, D, H * D, kind | (_lib.ROWS_PAIRED if pair else 0),
-                _lib.ptr(dst), D, rows_out * D, row_off, _lib.ptr(s), D // 128, (rows_out // 128) * (D // 128),
+                _lib.addr(src), _src_dtype(src), E, H, D, D, H * D, kind | (_lib.ROWS_PAIRED if pair else 0),
+                _lib.addr(dst), D, rows_out * D, row_off, _lib.addr(s), D // 128, (rows_out // 128) * (D // 128),
                 None, 0, 0, 0, None, 0, 0)
 
         jobs = (_lib.FmWeightJob * 3)(job(srcs[0], W13, S13, 0, 2 * H, paired),
@@ -810,9 +882,9 @@ class ExpertWeights:
         BF = _lib.QUANT_BF16
 
         def job(src, dst_t, col_off, cols_out):
-            return _lib.FmWeightJob(_lib.ptr(src), _lib.DTYPE_BF16, E, H, D, D, H * D, BF,
+            return _lib.FmWeightJob(_lib.addr(src), _lib.DTYPE_BF16, E, H, D, D, H * D, BF,
                                     None, 0, 0, 0, None, 0, 0,
-                                    _lib.ptr(dst_t), cols_out, D * cols_out, col_off, None, 0, 0)
+                                    _lib.addr(dst_t), cols_out, D * cols_out, col_off, None, 0, 0)
 
         jobs = [] if nn else [job(w2, W2t, 0, H)]
         if dgrad and not nn:
@@ -841,10 +913,10 @@ class ExpertWeights:
         MX = _lib.QUANT_MX
         # gate|up: w1 and w3 read in place as the [E, 2H, D] stack
         W13, S13, W13t, S13t = _alloc_quant(E * 2 * H, D, MX, True, dgrad, dev)
-        _lib.call("fm_quantize_pair", _lib.ptr(w1), _lib.ptr(w3), _src_dtype(w1), E, H, D, D,
+        _lib.call("fm_quantize_pair", _lib.addr(w1), _lib.addr(w3), _src_dtype(w1), E, H, D, D,
                   *_tile_args(MX, W13, S13, W13t, S13t, paired, paired and dgrad), stream)
         W2, S2, W2t, S2t = _alloc_quant(E * H, D, MX, dgrad, True, dev)
-        _lib.call("fm_quantize", _lib.ptr(w2), _src_dtype(w2), E * H, D, D,
+        _lib.call("fm_quantize", _lib.addr(w2), _src_dtype(w2), E * H, D, D,
                   *_tile_args(MX, W2, S2, W2t, S2t, paired and dgrad, paired), stream)
         cs = 2 if paired else 1   # column-offset group strides in a paired buffer
         self.w13 = ExpertWeightOperand(W13, S13, D, 2 * H * D, D // 32, 1, 2 * H * D // 32, 0, 2 * H, D,
@@ -869,6 +941,18 @@ def _side_stream(dev) -> torch.cuda.Stream:
     if s is None:
         s = _SIDE[idx] = torch.cuda.Stream(device=idx)
     return s
+
+
+# The router's backward runs on the second stream only where the expert outputs
+# it reads (T K rows) are at least this many bytes, or in a capture.  Issued
+# eagerly, the two stream waits and the stream switch cost the host 30-40 us a step
+# (1024 tokens, D 2048: 518 us a step with the second stream, 475 without; 3001:
+# 568 / 557), which larger steps gain back on the GPU (16384 tokens: 1301 / 1330).
+_ROUTER_BESIDE_BYTES = 32 << 20
+
+
+def _capturing() -> bool:
+    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
 
 
 # ================================================================ expert block ====
@@ -996,8 +1080,9 @@ class FP8FlowMoECompute:
         x2 = x.reshape(-1, shape[-1])
         K = indices.shape[-1]
         # the dgrad weight operands are built only for a forward that records a backward
-        self._record = torch.is_grad_enabled() and any(
-            t.requires_grad for t in (x, weights, *self._w))
+        w1, w2, w3 = self._w
+        self._record = torch.is_grad_enabled() and (x.requires_grad or weights.requires_grad or w1.requires_grad
+                                                    or w2.requires_grad or w3.requires_grad)
         out = _FlowMoEFunction.apply(x2, weights.reshape(-1, K), *self._w,
                                      indices.reshape(-1, K), self)
         return out.reshape(shape)
@@ -1051,28 +1136,25 @@ class FP8FlowMoECompute:
         if mask is not None:
             tiles[fp8_kind], tiles[_lib.QUANT_BF16] = plan.precision_tiles()
         saved = {}
-        pcols = {k: self._paired_cols(k, plan, mask) for k in kinds}
+        pcols = {k: self._paired_cols(k, plan, mask) for k in kinds} if self._record else {}
         for kind, want in ((fp8_kind, 1), (_lib.QUANT_BF16 if use_bf16 else None, 0)):
             if kind is None:
                 continue
             ew = ews[kind]
-            pt = fused_permute_pad(x, plan, E, granularity=_gran(kind), pow2_scale=kind == _lib.QUANT_POW2,
-                                   return_transpose=self._record, kmajor_scales=True,
-                                   tile_valid=tiles.get(kind, plan.tile_expert), paired_rows=self._paired(kind),
-                                   paired_cols=pcols.get(kind, False))
-            _gemm_m(kind, pt.rows, ew.w13, plan, GU, mask, want)
-            saved[kind] = (pt.rows_t, ew)
+            rows, cols = _permute_act(x, plan, kind, self._record, None, tiles.get(kind, plan.tile_expert),
+                                      self._paired(kind), pcols.get(kind, False))
+            _gemm_m(kind, rows, ew.w13, plan, GU, mask, want)
+            saved[kind] = (cols, ew)
         h_cols = {}
         for kind, want in ((fp8_kind, 1), (_lib.QUANT_BF16 if use_bf16 else None, 0)):
             if kind is None:
                 continue
             # row blocks feed the down GEMM; the column blocks are kept for dW2
-            pr = self._paired(kind)
-            pc = pcols[kind]
-            q, s, qt, st = _swiglu(GU[:, :H], GU[:, H:], R, H, kind, True, self._record, dev,
-                                   tiles.get(kind, plan.tile_expert), kmajor=True, paired=pr, col_paired=pc)
-            hrow, hcol = _wrap(q, s, qt, st, kind, pr, pc)
-            h_cols[kind] = hcol
+            hrow, h_cols[kind], args = _alloc_act(R, H, kind, self._record, dev, self._paired(kind),
+                                                  pcols.get(kind, False))
+            gu = GU.data_ptr()   # gate columns, then up columns (bf16)
+            _lib.call("fm_swiglu_quantize", gu, 2 * H, gu + 2 * H, 2 * H, R, H, *args,
+                      _lib.ptr(tiles.get(kind, plan.tile_expert)), _lib.stream_of(GU))
             _gemm_m(kind, hrow, saved[kind][1].w2t, plan, Y, mask, want)
         if self._dense:
             # the output must not be a view made inside this Function (callers
@@ -1125,8 +1207,8 @@ class FP8FlowMoECompute:
             dot = RouterDotInputs(dO, Y, plan.row_of)
         elif ctx.needs_input_grad[1]:
             dw = torch.empty(T * K, dtype=torch.float32, device=dev)
-            _lib.call("fm_router_weight_grad", _lib.ptr(dO), dO.stride(0), _lib.ptr(Y), Y.stride(0),
-                      _lib.ptr(plan.row_of), T, K, D, _lib.ptr(dw), _lib.stream_of(dO))
+            _lib.call("fm_router_weight_grad", _lib.addr(dO), dO.stride(0), _lib.addr(Y), Y.stride(0),
+                      _lib.addr(plan.row_of), T, K, D, _lib.addr(dw), _lib.stream_of(dO))
         main = torch.cuda.current_stream(dev)
         side = _side_stream(dev) if self.overlap_streams else main
         # the router's share of the input gradient: a [T, D] addend, or its
@@ -1134,9 +1216,15 @@ class FP8FlowMoECompute:
         # reads only dO, the saved expert outputs and x, so it runs on the second
         # stream beside the dY permute and dH; the unpermute waits for it.
         rshare = {}
+        used_side = False
         if on_router_grad is not None:
-            side.wait_stream(main)
-            with torch.cuda.stream(side):
+            beside = side is not main and (T * K * D * 2 >= _ROUTER_BESIDE_BYTES or _capturing())
+            if beside:
+                used_side = True
+                side.wait_stream(main)
+                with torch.cuda.stream(side):
+                    rshare = on_router_grad(None if dw is None else dw.reshape(T, K), not self._dense, dot)
+            else:
                 rshare = on_router_grad(None if dw is None else dw.reshape(T, K), not self._dense, dot)
         dH = torch.empty(R, H, dtype=torch.bfloat16, device=dev)
         dXp = torch.empty(R, D, dtype=torch.bfloat16, device=dev)
@@ -1149,17 +1237,15 @@ class FP8FlowMoECompute:
         runs = [(k, w) for k, w in ((fp8_kind, 1), (_lib.QUANT_BF16 if use_bf16 else None, 0)) if k is not None]
         tiles = ctx.tiles
         pcols = ctx.pcols
-        dy = {kind: fused_permute_pad(dO, plan, E, granularity=_gran(kind), pow2_scale=kind == _lib.QUANT_POW2,
-                                      return_transpose=True, weights=None if self._dense else wts,
-                                      kmajor_scales=True, tile_valid=tiles.get(kind, plan.tile_expert),
-                                      paired_rows=self._paired(kind), paired_cols=pcols.get(kind, False))
+        dy = {kind: _permute_act(dO, plan, kind, True, None if self._dense else wts,
+                                 tiles.get(kind, plan.tile_expert), self._paired(kind), pcols.get(kind, False))
               for kind, _ in runs}
         # dH and dW2 (contraction over each expert's tokens) both read the
         # permuted dY: each alone leaves its last round of workgroups
         # part-empty when the hidden size is not a multiple of the 256-wide
-        # tile.  One grid holds both (BF16, pow2) when dW2's tiles fill at
+        # tile.  One grid holds both (all but MX) when dW2's tiles fill at
         # least a round of the GPU's CUs; otherwise (a few long tiles, as for
-        # a shared expert's one group) and for the other kinds dW2 runs on the
+        # a shared expert's one group) and for MX dW2 runs on the
         # second stream beside dH and what follows it, with no K split (the
         # CUs it leaves idle run the main stream).  The forward's saved SwiGLU
         # columns are dW2's operand not in cache.
@@ -1169,28 +1255,26 @@ class FP8FlowMoECompute:
                     if k in _MK_KINDS and fill and (not self._paired(k) or pcols.get(k, False))]
         two_streams = [(k, w) for k, w in runs if (k, w) not in one_grid]
         if two_streams:
+            used_side = used_side or side is not main
             side.wait_stream(main)
             with torch.cuda.stream(side):
                 for kind, want in two_streams:
-                    _gemm_k(kind, ctx.saved_hcols[kind], dy[kind].rows_t, plan, H, D, dW2, H * D, mask=mask,
+                    _gemm_k(kind, ctx.saved_hcols[kind], dy[kind][1], plan, H, D, dW2, H * D, mask=mask,
                             want=want, may_split=side is main, a_cold=True)
         if ctx.dgrad_ops is None:
             raise RuntimeError("the expert block's forward did not record a backward")
         for kind, want in one_grid:
-            _gemm_mk(kind, dy[kind].rows, ctx.dgrad_ops[kind][0], plan, dH, ctx.saved_hcols[kind],
-                     dy[kind].rows_t, H, D, dW2, H * D, mask, want, a_cold=True)
+            _gemm_mk(kind, dy[kind][0], ctx.dgrad_ops[kind][0], plan, dH, ctx.saved_hcols[kind],
+                     dy[kind][1], H, D, dW2, H * D, mask, want, a_cold=True)
         for kind, want in two_streams:
-            _gemm_m(kind, dy[kind].rows, ctx.dgrad_ops[kind][0], plan, dH, mask, want)
+            _gemm_m(kind, dy[kind][0], ctx.dgrad_ops[kind][0], plan, dH, mask, want)
         if self.capture_intermediates is not None:
             self.capture_intermediates["dh"] = dH.detach().clone()
         for kind, want in runs:
-            pr = self._paired(kind)
-            pc = pcols.get(kind, False)
-            gq, gs, gqt, gst = _alloc_quant(R, 2 * H, kind, True, True, dev, kmajor=True)
-            _lib.call("fm_swiglu_backward", _lib.ptr(GU), GU.stride(0), _lib.ptr(GU[:, H:]), GU.stride(0),
-                      _lib.ptr(dH), dH.stride(0), R, H, *_tile_args(kind, gq, gs, gqt, gst, pr, pc),
+            dgu_row, dgu_col, args = _alloc_act(R, 2 * H, kind, True, dev, self._paired(kind), pcols.get(kind, False))
+            gu = GU.data_ptr()
+            _lib.call("fm_swiglu_backward", gu, 2 * H, gu + 2 * H, 2 * H, dH.data_ptr(), H, R, H, *args,
                       _lib.ptr(tiles.get(kind, plan.tile_expert)), _lib.stream_of(GU))
-            dgu_row, dgu_col = _wrap(gq, gs, gqt, gst, kind, pr, pc)
             # dW1 | dW3: contraction over each expert's tokens
             _gemm_k(kind, dgu_col, ctx.saved_cols[kind], plan, 2 * H, D, dW1, H * D, dW3, H * D, split=H,
                     mask=mask, want=want)
@@ -1198,7 +1282,8 @@ class FP8FlowMoECompute:
             _gemm_m(kind, dgu_row, ctx.dgrad_ops[kind][1], plan, dXp, mask, want)
         # the router's backward and dW2 (and the buffers they read, referenced
         # until here) are done before the router's dx share is summed
-        main.wait_stream(side)
+        if used_side:
+            main.wait_stream(side)
         dx_addend = rshare.get("addend")
         if self._dense:
             dx = dXp[:T] if dx_addend is None else dXp[:T] + dx_addend
@@ -1253,11 +1338,3 @@ class FP8SharedExpertCompute:
             r = self._route[key] = (torch.ones(T, 1, dtype=torch.float32, device=x.device),
                                     torch.zeros(T, 1, dtype=torch.int64, device=x.device))
         return self._block(x, r[0], r[1])
-
-
-def _gran(kind):
-    if kind == _lib.QUANT_BF16:
-        return None
-    if kind == _lib.QUANT_MX:
-        return G.MX_1x32
-    return G.ROW_1x128

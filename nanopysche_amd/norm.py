@@ -96,10 +96,10 @@ def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float = DEFAULT
     need_y = return_normed or (return_transpose and kind != _lib.QUANT_POW2)
     y = torch.empty(T, D, dtype=torch.bfloat16, device=dev) if need_y else None
     rstd = torch.empty(T, dtype=torch.float32, device=dev)
-    _lib.call("fm_rmsnorm_quantize", _lib.ptr(x2), _dtype_code(x2, "x"), x2.stride(0), T, D, _lib.ptr(w),
-              _dtype_code(w, "weight"), float(eps), _lib.ptr(y), 0 if y is None else y.stride(0), kind,
-              _lib.ptr(q), 0 if q is None else q.stride(0), _lib.ptr(s), 0 if s is None else s.stride(0),
-              _lib.ptr(rstd), _lib.stream_of(x2))
+    _lib.call("fm_rmsnorm_quantize", _lib.addr(x2), _dtype_code(x2, "x"), x2.stride(0), T, D, _lib.addr(w),
+              _dtype_code(w, "weight"), float(eps), _lib.addr(y), 0 if y is None else y.stride(0), kind,
+              _lib.addr(q), 0 if q is None else q.stride(0), _lib.addr(s), 0 if s is None else s.stride(0),
+              _lib.addr(rstd), _lib.stream_of(x2))
     rows = cols = None
     if kind != -1:
         rows = FP8Tensor(q, s, granularity, kind == _lib.QUANT_POW2)
@@ -130,12 +130,12 @@ def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, rs
         dw = torch.empty(D, dtype=weight.dtype, device=x.device)
         if T == 0:
             return dx.reshape(x.shape), dw.zero_()
-        nbytes = int(_lib.load().fm_rmsnorm_backward_workspace_bytes(T, D))
+        nbytes = _lib.size_of("fm_rmsnorm_backward_workspace_bytes", T, D)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
     w = weight if weight.is_contiguous() else weight.contiguous()
-    _lib.call("fm_rmsnorm_backward", _lib.ptr(dy2), dy2.stride(0), _lib.ptr(x2), _dtype_code(x2, "x"), x2.stride(0),
-              T, D, _lib.ptr(w), _dtype_code(w, "weight"), _lib.ptr(rstd), _lib.ptr(dx), dx.stride(0),
-              _lib.ptr(dw), 0 if dw is None else _dtype_code(dw, "weight"), _lib.ptr(ws), nbytes,
+    _lib.call("fm_rmsnorm_backward", _lib.addr(dy2), dy2.stride(0), _lib.addr(x2), _dtype_code(x2, "x"), x2.stride(0),
+              T, D, _lib.addr(w), _dtype_code(w, "weight"), _lib.addr(rstd), _lib.addr(dx), dx.stride(0),
+              _lib.addr(dw), 0 if dw is None else _dtype_code(dw, "weight"), _lib.addr(ws), nbytes,
               _lib.stream_of(x2))
     return dx.reshape(x.shape), dw
 

@@ -66,7 +66,7 @@ class RoutingPlan:
 
 def rows_max(num_assignments: int, num_experts: int) -> int:
     """Upper bound of the padded buffer's rows, known without reading counts."""
-    return int(_lib.load().fm_route_rows_max(num_assignments, num_experts))
+    return _lib.size_of("fm_route_rows_max", num_assignments, num_experts)
 
 
 def route_tokens(indices: torch.Tensor, num_experts: int, fp8_gemm_threshold: int = 0,
@@ -85,26 +85,24 @@ def route_tokens(indices: torch.Tensor, num_experts: int, fp8_gemm_threshold: in
     indices = indices.contiguous()
     T, K = indices.shape
     A = T * K
-    lib = _lib.load()
-    rmax = int(lib.fm_route_rows_max(A, num_experts))
+    rmax = rows_max(A, num_experts)
     dev = indices.device
-    i32 = dict(dtype=torch.int32, device=dev)
-    counts = torch.empty(num_experts, **i32)
-    offsets = torch.empty(num_experts + 1, **i32)
-    row_of = torch.empty(max(A, 1), **i32)
-    assign_of_row = torch.empty(rmax, **i32)
-    tile_expert = torch.empty(rmax // PAD_ROWS, **i32)
-    use_fp8 = torch.empty(num_experts, **i32)
-    ws_bytes = int(lib.fm_route_workspace_bytes(A, num_experts))
+    # the plan's arrays in one allocation, the ones read 16 bytes at a time first
+    E, pad = num_experts, (max(A, 1) + 3) // 4 * 4
+    row_of, assign_of_row, tile_expert, counts, offsets, use_fp8 = torch.empty(
+        pad + rmax + rmax // PAD_ROWS + 3 * E + 1, dtype=torch.int32, device=dev).split_with_sizes(
+            (pad, rmax, rmax // PAD_ROWS, E, E + 1, E))
+    ws_bytes = _lib.size_of("fm_route_workspace_bytes", A, E)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    args = (_lib.ptr(indices), int(indices.dtype == torch.int64), T, K, num_experts, int(fp8_gemm_threshold),
-            _lib.ptr(counts), _lib.ptr(offsets), _lib.ptr(row_of), _lib.ptr(assign_of_row), rmax,
-            _lib.ptr(tile_expert), _lib.ptr(use_fp8), _lib.ptr(ws), ws_bytes)
+    addr = _lib.addr
+    args = (addr(indices), int(indices.dtype == torch.int64), T, K, E, int(fp8_gemm_threshold),
+            addr(counts), addr(offsets), addr(row_of), addr(assign_of_row), rmax,
+            addr(tile_expert), addr(use_fp8), addr(ws), ws_bytes)
     if weight_jobs is None:
         _lib.call("fm_route_sort", *args, _lib.stream_of(indices))
     else:
         _lib.call("fm_route_sort_weights", *args, weight_jobs[0], weight_jobs[1], _lib.stream_of(indices))
-    return RoutingPlan(T, K, num_experts, rmax, counts, offsets, row_of[:A], assign_of_row,
+    return RoutingPlan(T, K, E, rmax, counts, offsets, row_of if pad == A else row_of[:A], assign_of_row,
                        tile_expert, use_fp8)
 
 
@@ -382,7 +380,7 @@ def router_forward(x2, gate_weight, gate_bias, score_bias, top_k, gating, replay
     idx = torch.empty(T, K, dtype=torch.int64, device=dev)
     counts = torch.empty(E, dtype=torch.int32, device=dev)
     aux = torch.empty((), dtype=torch.float32, device=dev)
-    ws = torch.empty(int(_lib.load().fm_router_forward_workspace_bytes(T, E)), dtype=torch.uint8, device=dev)
+    ws = torch.empty(_lib.size_of("fm_router_forward_workspace_bytes", T, E), dtype=torch.uint8, device=dev)
     rep = None
     if replay is not None:
         rep = replay.reshape(T, K)
@@ -392,11 +390,11 @@ def router_forward(x2, gate_weight, gate_bias, score_bias, top_k, gating, replay
     acc = tot = None
     if tracker is not None:
         acc, tot = tracker.tokens_per_expert, tracker.total_tokens
-    _lib.call("fm_router_forward", _lib.ptr(x2), _x_dtype(x2), x2.stride(0), T, D, _lib.ptr(w_), _dt_code(w_),
-              w_.stride(0), _lib.ptr(b), _lib.ptr(sb), E, K, _gating_code(gating), _norm_flags(normalize),
-              _lib.ptr(rep), int(rep is not None and rep.dtype == torch.int64), _lib.ptr(logits), logits.stride(0),
-              _lib.ptr(w), _lib.ptr(idx), 1, _lib.ptr(counts), _lib.ptr(acc), _lib.ptr(tot), float(z_mult),
-              _lib.ptr(aux), _lib.ptr(ws), ws.numel(), _lib.stream_of(x2))
+    _lib.call("fm_router_forward", _lib.addr(x2), _x_dtype(x2), x2.stride(0), T, D, _lib.addr(w_), _dt_code(w_),
+              w_.stride(0), _lib.addr(b), _lib.addr(sb), E, K, _gating_code(gating), _norm_flags(normalize),
+              _lib.addr(rep), int(rep is not None and rep.dtype == torch.int64), _lib.addr(logits), logits.stride(0),
+              _lib.addr(w), _lib.addr(idx), 1, _lib.addr(counts), _lib.addr(acc), _lib.addr(tot), float(z_mult),
+              _lib.addr(aux), _lib.addr(ws), ws.numel(), _lib.stream_of(x2))
     state = RouterState(logits, idx, counts, _gating_code(gating), _norm_flags(normalize), replay is not None,
                         float(z_mult))
     return w, idx, aux, state
@@ -430,27 +428,27 @@ def router_backward(state: RouterState, x2, gate_weight, dweights, daux, need_x=
     da = None if daux is None else daux.reshape(1).float().contiguous()
     dlogits = torch.empty(T, E, dtype=torch.float32, device=dev)
     if dot is not None:
-        _lib.call("fm_gating_grad_dot", _lib.ptr(logits), T, E, logits.stride(0), K, state.gating, state.flags,
-                  int(state.replay), _lib.ptr(idx), int(idx.dtype == torch.int64), None, _lib.ptr(dot.dout),
-                  dot.dout.stride(0), _lib.ptr(dot.y), dot.y.stride(0), _lib.ptr(dot.row_of), D, None, _lib.ptr(da),
-                  _lib.ptr(state.counts), state.z_mult, _lib.ptr(dlogits), dlogits.stride(0), st)
+        _lib.call("fm_gating_grad_dot", _lib.addr(logits), T, E, logits.stride(0), K, state.gating, state.flags,
+                  int(state.replay), _lib.addr(idx), int(idx.dtype == torch.int64), None, _lib.addr(dot.dout),
+                  dot.dout.stride(0), _lib.addr(dot.y), dot.y.stride(0), _lib.addr(dot.row_of), D, None, _lib.addr(da),
+                  _lib.addr(state.counts), state.z_mult, _lib.addr(dlogits), dlogits.stride(0), st)
     elif dwts is None and da is None:
         dlogits.zero_()
     else:
-        _lib.call("fm_gating_grad", _lib.ptr(logits), T, E, logits.stride(0), K, state.gating, state.flags,
-                  int(state.replay), _lib.ptr(idx), int(idx.dtype == torch.int64), _lib.ptr(dwts), _lib.ptr(da),
-                  _lib.ptr(state.counts), state.z_mult, _lib.ptr(dlogits), dlogits.stride(0), st)
+        _lib.call("fm_gating_grad", _lib.addr(logits), T, E, logits.stride(0), K, state.gating, state.flags,
+                  int(state.replay), _lib.addr(idx), int(idx.dtype == torch.int64), _lib.addr(dwts), _lib.addr(da),
+                  _lib.addr(state.counts), state.z_mult, _lib.addr(dlogits), dlogits.stride(0), st)
     w, _, _ = _gate_params(gate_weight, None, None)
     dx = torch.empty_like(x2) if need_x else None
     dW = torch.empty(E, D, dtype=w.dtype, device=dev) if need_w else None
     db = torch.empty(E, dtype=bias_dtype or torch.float32, device=dev) if need_b else None
     if dx is not None or dW is not None or db is not None:
-        ws = torch.empty(int(_lib.load().fm_router_workspace_bytes(T, D, E)), dtype=torch.uint8, device=dev)
-        _lib.call("fm_router_backward", _lib.ptr(dlogits), dlogits.stride(0), _lib.ptr(x2), _x_dtype(x2),
-                  x2.stride(0), T, D, _lib.ptr(w), _dt_code(w), w.stride(0), E, _lib.ptr(dx),
-                  0 if dx is None else dx.stride(0), _lib.ptr(dW), _lib.DTYPE_F32 if dW is None else _dt_code(dW),
-                  0 if dW is None else dW.stride(0), _lib.ptr(db), _lib.DTYPE_F32 if db is None else _dt_code(db),
-                  _lib.ptr(ws), ws.numel(), st)
+        ws = torch.empty(_lib.size_of("fm_router_workspace_bytes", T, D, E), dtype=torch.uint8, device=dev)
+        _lib.call("fm_router_backward", _lib.addr(dlogits), dlogits.stride(0), _lib.addr(x2), _x_dtype(x2),
+                  x2.stride(0), T, D, _lib.addr(w), _dt_code(w), w.stride(0), E, _lib.addr(dx),
+                  0 if dx is None else dx.stride(0), _lib.addr(dW), _lib.DTYPE_F32 if dW is None else _dt_code(dW),
+                  0 if dW is None else dW.stride(0), _lib.addr(db), _lib.DTYPE_F32 if db is None else _dt_code(db),
+                  _lib.addr(ws), ws.numel(), st)
     return dx, dW, db, dlogits
 
 
