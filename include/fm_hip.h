@@ -500,7 +500,7 @@ int fm_swiglu_values(const void* g, int64_t ld_g, const void* u, int64_t ld_u, c
  * pitch and group stride: rows r >= split_rows are row r - split_rows of
  * data2 -- the weights of fm_grouped_gemm_ragged_m read from w1 and w3 as
  * they are stored, without stacking them.  BF16 weights only, at most 64
- * experts; split_rows a multiple of 256 inside N, or, with FM_GEMM_W_KMAJOR
+ * experts; split_rows a multiple of 128 inside N, or, with FM_GEMM_W_KMAJOR
  * (rows are K rows), a multiple of 64 inside K. */
 typedef struct FmGemmOperand {
   const void* data;

@@ -1111,8 +1111,11 @@ __device__ __forceinline__ TileStreams tile_streams(const Operand& Q, const Oper
     } else {
       s.q = make_stream_nn(Q.p + int64_t(t.e) * Q.gs + int64_t(t.i0), Q.ld, lane, w.wave);
     }
-  } else {   // a tile lies in one of the two tensors of a split operand (split % 256 == 0)
-    const bool second = t.i0 >= Q.split;
+  } else {
+    // the two tensors of a split operand meet at a multiple of 128 rows: each of
+    // the tile's 128-row halves (waves 0-3, 4-7) lies in one of them
+    const int64_t half = w.wave >= 4 && q_rows > 128 ? 128 : 0;
+    const bool second = uniform_ge(t.i0 + half, Q.split);
     const int64_t qi = second ? t.i0 - Q.split : t.i0;
     s.q = make_stream((second ? Q.p2 : Q.p) + (int64_t(t.e) * Q.gs + qi * Q.ld) * ES, Q.ld * ES, q_rows, lane,
                       w.wave);
@@ -2649,9 +2652,9 @@ int ragged_m_params(int kind, int nn, int paired, const FmGemmOperand* tokens, c
   FM_REQUIRE(weights->data2 == nullptr ||
                  (kind == GK_BF16 && E <= 64 && K >= 128 && weights->split_rows > 0 &&
                   (nn ? weights->split_rows % 64 == 0 && weights->split_rows < K
-                      : weights->split_rows % 256 == 0 && weights->split_rows < N)),
+                      : weights->split_rows % 128 == 0 && weights->split_rows < N)),
              "fm_grouped_gemm_ragged_m: split weights need the BF16 kind, E <= 64, K >= 128 and a split that is "
-             "a multiple of 256 inside N ([K][N] weights: of 64 inside K)");
+             "a multiple of 128 inside N ([K][N] weights: of 64 inside K)");
   if (int rc = check_scale_span(*tokens, kind, m_tiles * 128, K, "tokens")) return rc;
   if (int rc = check_scale_span(*weights, kind, N, K, "weights")) return rc;
   FM_REQUIRE(N > 0 && N % 128 == 0, "fm_grouped_gemm_ragged_m: N must be a positive multiple of 128 (got %lld)", (long long)N);
