@@ -539,6 +539,17 @@ int fm_grouped_gemm_ragged_k(int kind, const FmGemmOperand* a_t, const FmGemmOpe
                              void* out2, int64_t out2_gs, int64_t split_rows, int out_dtype,
                              int64_t ld_out, void* stream);
 
+/* fm_grouped_gemm_ragged_m for BF16 and few tokens per expert (reference
+ * model/moe.py:1588-1591 at decoding sizes): rows [offsets[e], + counts[e]) of
+ * each group are multiplied, the group's remaining rows written as zeros (the
+ * product of the zero padding rows); an expert without tokens reads no weights.
+ * weights_kn: the weights stored [K][N].  N, K and split_rows multiples of 64,
+ * pitches of 8, 16-byte aligned buffers.  Any counts are computed (32 tokens a
+ * pass); past some tens of tokens per expert fm_grouped_gemm_ragged_m is faster. */
+int fm_grouped_gemm_few(const FmGemmOperand* tokens, const FmGemmOperand* weights, int weights_kn,
+                        const int32_t* counts, const int32_t* offsets, int E, int64_t N, int64_t K, void* out,
+                        int out_dtype, int64_t ld_out, void* stream);
+
 /* fm_grouped_gemm_ragged_m followed by fm_grouped_gemm_ragged_k on the same
  * stream, with the same offsets, E and expert mask, as one grid: for a
  * backward's dgrad dH = dY w2_e (reference model/moe.py:1588-1591, the bmm's

@@ -20,7 +20,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libfm_hip.so"
 SOURCES = ["fm_api.cpp", "fm_quant.hip", "fm_route.hip", "fm_swiglu.hip", "fm_gemm.hip", "fm_router.hip",
-           "fm_norm.hip"]
+           "fm_norm.hip", "fm_few.hip"]
 ARCH = "gfx950"
 
 

@@ -518,12 +518,39 @@ def _assignments(plan: RoutingPlan, mask, want) -> float:
     return float((plan.counts.to(torch.int64) * sel).sum().item())
 
 
+# BF16 ragged-M launches of few tokens take the kernel that streams each weight
+# row once per 32 tokens of its expert: at most 32 assignments per expert, and at
+# most 64 tokens (128 where an expert's operand is small enough to stay cached
+# between an expert's passes), so that an expert that all of them choose streams
+# its weights two (four) times.  Measured, that kernel against the 256-row tile,
+# gate|up / down us: 8 experts of 2048 x 1408, top-2: 16 tokens 17 / 11 against
+# 40 / 29, 128 tokens 26 / 15 against 40 / 29, 256 tokens 40 / 23 and 512 tokens
+# 71 / 39 against 41 / 30; 64 experts top-6, 128 tokens 148 / 89 against 216 / 98;
+# 8 of 4096 x 14336, 64 tokens 361 / 192 against 457 / 351, 128 tokens 479 / 317
+# against 458 / 351.  All tokens on the same experts: 8 of 2048 x 1408, 128 tokens
+# 25 / 23 against 36 / 28; 8 of 4096 x 14336, 64 tokens 153 / 94 against 122 / 229,
+# 128 tokens 274 / 178 against 135 / 229.
+_FEW_TOKENS = 128
+_FEW_PER_EXPERT = 32
+_FEW_CACHED_BYTES = 48 << 20
+
+
+def _few(plan: RoutingPlan, w) -> bool:
+    most = _FEW_TOKENS if w.N * w.K * 2 <= _FEW_CACHED_BYTES else _FEW_TOKENS // 2
+    return plan.num_tokens <= most and plan.num_tokens * plan.top_k <= _FEW_PER_EXPERT * plan.num_experts
+
+
 def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=None, want=1):
     t_paired = getattr(tokens, "paired", False)
     if (w.paired and not w.kmajor) and not t_paired:
         raise ValueError("paired-row weights need paired-row tokens")
 
     def launch():
+        if kind == _lib.QUANT_BF16 and mask is None and _few(plan, w):
+            _lib.call("fm_grouped_gemm_few", _token_operand(tokens, kind), w.operand(), int(w.kmajor),
+                      _lib.addr(plan.counts), _lib.addr(plan.offsets), plan.num_experts, w.N, w.K, _lib.addr(out),
+                      _dt(out), out.stride(0), _lib.stream_of(out))
+            return
         gk = _gemm_kind(kind) | (_lib.GEMM_W_KMAJOR if w.kmajor else 0)
         if t_paired:
             gk |= _lib.GEMM_PAIRED | (_lib.GEMM_W_PAIRED if w.kmajor and w.paired else 0)
