@@ -535,9 +535,25 @@ _FEW_PER_EXPERT = 32
 _FEW_CACHED_BYTES = 48 << 20
 
 
-def _few(plan: RoutingPlan, w) -> bool:
+def _few(plan: RoutingPlan, tokens, w, out) -> bool:
+    """Whether a BF16 launch takes fm_grouped_gemm_few: few tokens, in a form that both
+    entries take (what fm_grouped_gemm_ragged_m refuses goes there to be refused)."""
     most = _FEW_TOKENS if w.N * w.K * 2 <= _FEW_CACHED_BYTES else _FEW_TOKENS // 2
-    return plan.num_tokens <= most and plan.num_tokens * plan.top_k <= _FEW_PER_EXPERT * plan.num_experts
+    if plan.num_tokens > most or plan.num_tokens * plan.top_k > _FEW_PER_EXPERT * plan.num_experts:
+        return False
+    t = tokens.buf if type(tokens) is _Act else tokens
+    ld = tokens.ld if type(tokens) is _Act else tokens.stride(0)
+    if w.N % 128 or w.K % 128 or w.ld % 16 or w.gs % 8 or w.gs < w.K or ld % 16 or ld < w.K or plan.rows_max == 0:
+        return False
+    if (w.kmajor or w.data2 is not None) and plan.num_experts > 64:
+        return False
+    if w.kmajor and (w.N % 256 or w.ld < w.N or w.gs < w.ld * (w.K if w.data2 is None else 1)):
+        return False
+    if w.data2 is not None and (w.split % (64 if w.kmajor else 128) or not 0 < w.split < (w.K if w.kmajor else w.N)):
+        return False
+    return (out.stride(0) % 8 == 0 and out.stride(0) >= w.N and not w.paired
+            and not (t.data_ptr() | w.data.data_ptr() | out.data_ptr()
+                     | (0 if w.data2 is None else w.data2.data_ptr())) & 15)
 
 
 def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=None, want=1):
@@ -546,7 +562,7 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
         raise ValueError("paired-row weights need paired-row tokens")
 
     def launch():
-        if kind == _lib.QUANT_BF16 and mask is None and _few(plan, w):
+        if kind == _lib.QUANT_BF16 and mask is None and _few(plan, tokens, w, out):
             _lib.call("fm_grouped_gemm_few", _token_operand(tokens, kind), w.operand(), int(w.kmajor),
                       _lib.addr(plan.counts), _lib.addr(plan.offsets), plan.num_experts, w.N, w.K, _lib.addr(out),
                       _dt(out), out.stride(0), _lib.stream_of(out))

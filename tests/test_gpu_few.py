@@ -79,3 +79,25 @@ def test_small_block_against_larger_tile(dev, H, monkeypatch):
         got.append((out.detach(), *torch.autograd.grad(out, t, torch.ones_like(out))))
     for a, b in zip(*got):
         assert (a.double() - b.double()).norm() <= 4e-3 * b.double().norm() + 1e-30
+
+
+def test_forms_outside_the_rule_keep_their_kernel(dev, monkeypatch):
+    """Pitches and alignments that only the tile entry takes go there, and what it refuses stays refused."""
+    E, N, K = 2, 128, 128
+    idx = torch.tensor([[0], [1], [1]], device=dev)
+    plan = fm.route_tokens(idx, E)
+    tokens = randn_bf16((plan.rows_max, K), seed=1).to(dev)
+    W = randn_bf16((E, N, K), seed=2).to(dev)
+    w = ExpertWeightOperand(W, None, K, N * K, N=N, K=K)
+    ref = fm.fp8_grouped_gemm(tokens, w, plan)
+    called, real = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    wide = torch.zeros(plan.rows_max, N + 4, dtype=torch.bfloat16, device=dev)[:, :N]     # pitch 4 mod 8
+    got = fm.fp8_grouped_gemm(tokens, w, plan, out=wide)
+    assert called == ["fm_grouped_gemm_ragged_m"]
+    for e, c in enumerate((1, 2)):
+        r = int(plan.offsets[e])
+        assert (got[r:r + c].double() - ref[r:r + c].double()).norm() <= 4e-3 * ref[r:r + c].double().norm()
+    narrow = ExpertWeightOperand(W[:, :64].contiguous(), None, K, 64 * K, N=64, K=K)
+    with pytest.raises(RuntimeError, match="multiple of 128"):
+        fm.fp8_grouped_gemm(tokens, narrow, plan)
