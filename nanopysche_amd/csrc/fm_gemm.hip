@@ -2328,6 +2328,214 @@ __global__ __launch_bounds__(512) void gemm256r_kernel(GemmParams pm, GemmParams
 }
 
 // ============================================================================
+// Ragged-K tiles of few K steps (weight gradients of experts with few tokens)
+// ============================================================================
+// An expert with few tokens gives each output tile only a few K steps, and the
+// launch is bound by writing the gradients.  A persistent 256 x 256 walk keeps
+// one workgroup per CU, whose operand loads queue behind its own output stores
+// (vector memory operations of a wave complete in order): the CU's store drain,
+// load latency and matrix work follow one another.  Here a workgroup is four
+// waves on a 128 x 128 tile with one 32 KiB stage, four of them to a CU, so
+// that one loads or computes while another's stores drain; a workgroup ends
+// without waiting for its stores.  Measured on the 256 x 256 tiles before and
+// here, experts of 4096 x 14336 with about 300 tokens (bf16) or 1000 (pow2), some
+// masked out: dW1 | dW3 655 -> 522 us and 502 -> 395 us.  What bounds it is the
+// operand stream (2 x 16 KiB a step, 6.8 TB/s over the chip) with the loads of
+// about half of the workgroups in flight.
+// The waves are 2 (i) x 2 (j) of 64 x 64.  Every XCD takes blocks of 64
+// consecutive tiles (8 i x 8 j, which share operand rows in its L2).  Fragments
+// and the MFMA order are those of the 256 x 256 kernels: the same bits.
+constexpr int kTS = 128;
+constexpr int kShortChunk = 64;
+
+template <int KIND>
+struct FragS {
+  v8i a[2], b[2];
+};
+template <>
+struct FragS<GK_BF16> {
+  v8bf a[2], b[2];
+};
+
+template <int KIND, bool PAIRED>
+__global__ __launch_bounds__(256, 4) void gemm128k_kernel(GemmParams p) {
+  static_assert(KIND == GK_FP8_POW2 || (KIND == GK_BF16 && !PAIRED), "bf16, or pow2 in either layout");
+  constexpr bool SC = KIND != GK_BF16;
+  constexpr int ES = KIND == GK_BF16 ? 2 : 1;
+  constexpr int KSTEP = 128 / ES;
+  constexpr int kOp = kTS * 128;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kOp + (SC ? 2 * kTS * 4 : 0)];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int wi = wave >> 1, wj = wave & 1, lrow = lane & 31, lhalf = lane >> 5;
+
+  // the tile: the experts this launch runs, in order, NI x NJ tiles each
+  const bool run = lane < p.E && (p.mask == nullptr || p.mask[lane < p.E ? lane : 0] == p.mask_want);
+  const unsigned long long act = __ballot(run);
+  const int NI = int(p.n_i / kTS), NJ = int(p.n_j / kTS), per_e = NI * NJ;
+  const int loc = int(blockIdx.x >> 3);
+  const int L = ((loc / kShortChunk) * 8 + int(blockIdx.x & 7)) * kShortChunk + loc % kShortChunk;
+  if (L >= __popcll(act) * per_e) return;
+  const int rank = L / per_e, Lr = L - rank * per_e;
+  const unsigned long long below = act & ((1ull << lane) - 1);
+  const int e = __builtin_amdgcn_readfirstlane(__ffsll(__ballot(run && __popcll(below) == rank)) - 1);
+  const int group = Lr / (kGroupM * NJ), first = group * kGroupM;
+  const int gsz = NI - first < kGroupM ? NI - first : kGroupM;
+  const int rem = Lr - group * kGroupM * NJ;
+  const int64_t i0 = int64_t(first + rem % gsz) * kTS, j0 = int64_t(rem / gsz) * kTS;
+  const int64_t k_lo = __builtin_amdgcn_readfirstlane(p.offsets[e]);
+  const int nk = (__builtin_amdgcn_readfirstlane(p.offsets[e + 1]) - int(k_lo)) / KSTEP;
+
+  const uint32_t lds = lds_addr(smem);
+  OpStream qs, ps;
+  RingStream qr, pr;
+  if constexpr (PAIRED) {
+    qr = make_stream_pr(p.Q.p + i0 * p.Q.ld, p.Q.ld, kTS, lane, wave);
+    pr = make_stream_pr(p.P.p + j0 * p.P.ld, p.P.ld, kTS, lane, wave);
+  } else {
+    qs = make_stream(p.Q.p + i0 * p.Q.ld * ES, p.Q.ld * ES, kTS, lane, wave);
+    ps = make_stream(p.P.p + j0 * p.P.ld * ES, p.P.ld * ES, kTS, lane, wave);
+  }
+  // pow2 scales: waves 0-1 stream Q's, 2-3 P's; slot li of an operand holds
+  // tile row 64 (li / 64) + 32 (li % 2) + (li % 64) / 2, so a lane's two row
+  // blocks come from one 8-byte read
+  v4i srsrc;
+  uint32_t svoff = 0, sk = 0;
+  if constexpr (SC) {
+    const bool wq = wave < 2;
+    const int li = int(threadIdx.x) & 127;
+    const int64_t row = (wq ? i0 : j0) + (li >> 6) * 64 + (li & 1) * 32 + ((li & 63) >> 1);
+    srsrc = make_rsrc(wq ? p.Q.s : p.P.s);
+    svoff = uint32_t((row >> (wq ? p.Q.s_shift : p.P.s_shift)) * (wq ? p.Q.s_row : p.P.s_row) * 4);
+    sk = uint32_t((wq ? p.Q.s_kb : p.P.s_kb) * 4);
+  }
+  auto issue = [&](int t) {
+    const uint32_t k = uint32_t(k_lo) + uint32_t(t) * KSTEP;
+    if constexpr (PAIRED) {
+      // half h of an operand's stage at h * 8 KiB
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const uint32_t kb = (k / 64 + h) * 128, dst = lds + h * (kOp / 2) + (wave * 2 + g) * 1024;
+          bdma16(qr.rsrc, qr.lane_off[g], g * qr.group_bytes + kb, dst);
+          bdma16(pr.rsrc, pr.lane_off[g], g * pr.group_bytes + kb, dst + kOp);
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t dst = lds + (wave * 4 + u) * 1024;
+        bdma16(qs.rsrc, qs.lane_off[u & 1], u * qs.group_bytes + k * ES, dst);
+        bdma16(ps.rsrc, ps.lane_off[u & 1], u * ps.group_bytes + k * ES, dst + kOp);
+      }
+    }
+    if constexpr (SC) bdma4(srsrc, svoff, (k / KSTEP) * sk, lds + 2 * kOp + wave * 256);
+  };
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+#pragma unroll 1
+  for (int t = 0; t < nk; ++t) {
+    if (t > 0) block_barrier();   // every wave has read step t - 1 (its MFMAs consumed the fragments)
+    issue(t);
+    FM_WAIT_VMCNT(0);
+    block_barrier();
+    if constexpr (KIND == GK_BF16) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        FragS<KIND> f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f.a[u] = read_frag16(smem, wi * 64 + u * 32 + lrow, ks, lhalf);
+          f.b[u] = read_frag16(smem + kOp, wj * 64 + u * 32 + lrow, ks, lhalf);
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[a], f.b[b], acc[a][b], 0, 0, 0);
+      }
+    } else {
+      const uint8_t* sc = smem + 2 * kOp;
+      const uint2 vq = *reinterpret_cast<const uint2*>(sc + wi * 256 + lrow * 8);
+      const uint2 vp = *reinterpret_cast<const uint2*>(sc + kTS * 4 + wj * 256 + lrow * 8);
+      const int sa = pack_exp4(vq.x, vq.y, 0u, 0u), sb = pack_exp4(vp.x, vp.y, 0u, 0u);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        FragS<KIND> f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int ra = wi * 64 + u * 32 + lrow, rb = wj * 64 + u * 32 + lrow;
+          if constexpr (PAIRED) {
+            f.a[u] = read_frag8_pr(smem + h * (kOp / 2), ra, lhalf);
+            f.b[u] = read_frag8_pr(smem + kOp + h * (kOp / 2), rb, lhalf);
+          } else {
+            f.a[u] = read_frag8(smem, ra, h, lhalf);
+            f.b[u] = read_frag8(smem + kOp, rb, h, lhalf);
+          }
+        }
+        acc[0][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[0], f.b[0], acc[0][0], 0, 0, 0, sa, 0, sb);
+        acc[0][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[0], f.b[1], acc[0][1], 0, 0, 0, sa, 1, sb);
+        acc[1][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[1], f.b[0], acc[1][0], 0, 0, 1, sa, 0, sb);
+        acc[1][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[1], f.b[1], acc[1][1], 0, 0, 1, sa, 1, sb);
+      }
+    }
+  }
+
+  // output row j, contiguous column i; each wave turns its 64 x 64 block
+  // around in its own 8 KiB of the stage and writes whole row segments
+  const int64_t ib = i0 + wi * 64, jb = j0 + wj * 64;
+  const bool second = uniform_ge(jb, p.split);
+  const int64_t off = int64_t(e) * (second ? p.c2_gs : p.c_gs) + (second ? jb - p.split : jb) * p.ldC + ib;
+  void* const C = second ? p.C2 : p.C;
+  uint8_t* const W = smem + wave * 8192;
+  block_barrier();   // every wave has read the last step
+  if (!p.out_f32) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int jr = b * 32 + lrow;
+          *reinterpret_cast<uint2*>(W + jr * 128 + (((a * 4 + q) ^ (jr & 7)) << 4) + lhalf * 8) =
+              make_uint2(hw_bf16x2(acc[a][b][4 * q], acc[a][b][4 * q + 1]),
+                         hw_bf16x2(acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]));
+        }
+    const int c = lane & 7;
+    uint16_t* const dst = static_cast<uint16_t*>(C) + off + c * 8;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const int rr = n * 8 + (lane >> 3);
+      st_global(dst + rr * p.ldC, *reinterpret_cast<const uint4*>(W + rr * 128 + ((c ^ (rr & 7)) << 4)));
+    }
+  } else {
+    const int c = lane & 15;
+    float* const dst = static_cast<float*>(C) + off + c * 4;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {   // 32 rows x 256 bytes a pass
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(W + lrow * 256 + (((a * 8 + 2 * q + lhalf) ^ (lrow & 15)) << 4)) =
+              make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        const int rr = n * 4 + (lane >> 4);
+        st_global(dst + (b * 32 + rr) * p.ldC,
+                  *reinterpret_cast<const float4*>(W + rr * 256 + ((c ^ (rr & 15)) << 4)));
+      }
+    }
+  }
+}
+
+// ============================================================================
 // launch
 // ============================================================================
 // FM_RK_XCD=0: ragged-K launches keep their tiles in launch order even for
@@ -2505,6 +2713,36 @@ int prepare_gemm(int kind, GemmParams& p) {
   return 0;
 }
 
+// Ragged-K launches of few tokens per expert take the 128 x 128 kernel: at most
+// 512 padded tokens an expert on average, or 1152 where an expert's gradient has
+// 2^25 elements or more (`p` as prepared; the operands' pitch bounds the tokens).
+// Measured over a training step, 256 x 256 kernels against this one, at 128 /
+// 256 / 384 / 512 / 1024 tokens per expert: 8 experts of 4096 x 14336 (pow2) 2553
+// / 2826 / 3155 / 3886 / 5711 us against 2409 / 2659 / 3030 / 3727 / 5536 (bf16
+// 3327 / 3930 / 4492 / 6269 / 10493 against 3109 / 3756 / 4288 / 6192 / 10234), 8
+// experts of 2048 x 1408 (pow2) 286 / 301 / 325 / 330 / 469 against 271 / 286 /
+// 316 / 345 / 485, 64 such experts (bf16) 1399 / 1934 / 2288 / 2682 / 4587 against
+// 1320 / 1852 / 2285 / 2632 / 4589.  The larger tiles reuse operands better, which
+// counts from about 512 tokens on, later where the operands of an expert's tiles
+// in flight leave an XCD's L2 either way.
+constexpr int64_t kShortRows = 512, kShortRowsLarge = 1152, kShortLarge = int64_t(1) << 25;
+inline bool gemm_rk_short(int kind, const GemmParams& p) {
+  const int64_t row = p.out_f32 ? 4 : 8;   // elements of a 16-byte store
+  const bool aligned = p.ldC % row == 0 && p.c_gs % row == 0 && (size_t(p.C) & 15) == 0 &&
+                       (p.split == INT64_MAX || (p.c2_gs % row == 0 && (size_t(p.C2) & 15) == 0));
+  const int64_t rows = p.n_i * p.n_j >= kShortLarge ? kShortRowsLarge : kShortRows;
+  return (kind == GK_BF16 || kind == GK_FP8_POW2) && p.splits == 1 && p.E <= 64 && aligned &&
+         p.P.ld <= rows * p.E && p.n_tiles < (int64_t(1) << 24);
+}
+inline void launch128k(int kind, const GemmParams& p, hipStream_t s) {
+  const int64_t tiles = int64_t(p.E) * (p.n_i / kTS) * (p.n_j / kTS);
+  const int64_t chunks = (tiles + kShortChunk - 1) / kShortChunk;
+  const dim3 grid(unsigned((chunks + 7) / 8 * 8 * kShortChunk)), block(256);
+  if (kind == GK_BF16) hipLaunchKernelGGL((gemm128k_kernel<GK_BF16, false>), grid, block, 0, s, p);
+  else if (p.paired) hipLaunchKernelGGL((gemm128k_kernel<GK_FP8_POW2, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm128k_kernel<GK_FP8_POW2, false>), grid, block, 0, s, p);
+}
+
 template <int MODE>
 int dispatch_gemm(int kind, GemmParams p, hipStream_t s) {
   if (int rc = prepare_gemm<MODE>(kind, p)) return rc;
@@ -2515,6 +2753,8 @@ int dispatch_gemm(int kind, GemmParams p, hipStream_t s) {
   } else if (MODE == GM_RAGGED_M && p.E <= 64 && p.K / (kind == GK_BF16 ? 64 : 128) >= 2 &&
              (gemm_persistent() || p.q_nn || p.paired || p.Q.split != INT64_MAX)) {
     launch256p(kind, p, s);
+  } else if (MODE == GM_RAGGED_K && gemm_rk_short(kind, p)) {
+    launch128k(kind, p, s);
   } else if (MODE == GM_RAGGED_K && p.paired) {
     // paired-row operands (checked by the entry point): the ring walk
     const int64_t slots = int64_t(device_cus() / 8 > 0 ? device_cus() / 8 : 1) * 8;
@@ -2804,6 +3044,9 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
     return rc;
   pk.rk_jfast = a_fast;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  GemmParams pks = pk;
+  if (int rc = prepare_gemm<GM_RAGGED_K>(kind, pks)) return rc;
+  const bool rk_short = gemm_rk_short(kind, pks);   // a kernel of its own beats the shared grid
   if (paired) {
     // every operand paired: one ring walk over the dgrad tiles, then the weight-gradient tiles
     FM_REQUIRE(!nn && expert_mask == nullptr && a_t->ld % 64 == 0 && b_t->ld % 64 == 0 &&
@@ -2811,7 +3054,7 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
                "fm_grouped_gemm_ragged_m_k: paired-row operands need [N][K] weights, no expert mask, "
                "pitches that are multiples of 64 and fewer than 2^28 weight-gradient tiles");
     pk.paired = 1;
-    if (kind != GK_FP8_POW2) {   // MX: the two ring launches (one grid would need both MX scale layouts)
+    if (kind != GK_FP8_POW2 || rk_short) {   // MX: two ring launches (one grid would need both MX scale layouts)
       if (pm.m_tiles > 0)
         if (int rc = dispatch_gemm<GM_RAGGED_M>(kind, pm, s)) return rc;
       return dispatch_gemm<GM_RAGGED_K>(kind, pk, s);
@@ -2826,7 +3069,7 @@ int fm_grouped_gemm_ragged_m_k(int kind, const FmGemmOperand* tokens, const FmGe
     else hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_POW2, 0, true, true, false, true>), pgrid, pblock, 0, s, pm, pk);
     return check_launch("fm_grouped_gemm_ragged_m_k");
   }
-  if (nn || pm.m_tiles == 0 || kind == GK_FP8_MX || !gemm_mk_one_grid()) {
+  if (nn || pm.m_tiles == 0 || kind == GK_FP8_MX || rk_short || !gemm_mk_one_grid()) {
     if (pm.m_tiles > 0)
       if (int rc = dispatch_gemm<GM_RAGGED_M>(kind, pm, s)) return rc;
     return dispatch_gemm<GM_RAGGED_K>(kind, pk, s);
