@@ -143,6 +143,8 @@ SIGNATURES = {
     "fm_swiglu_values": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "fm_grouped_gemm_ragged_m": (_i32, [_i32, _OPND, _OPND, _i64, _vp, _vp, _i32, _i64, _i64, _vp,
                                         _i32, _vp, _i32, _i64, _vp]),
+    "fm_grouped_gemm_ragged_m_split": (_i32, [_i32, _OPND, _OPND, _i64, _vp, _vp, _i32, _i64, _i64, _vp, _i32, _vp,
+                                              _i64, _vp, _i64, _vp]),
     "fm_grouped_gemm_few": (_i32, [_OPND, _OPND, _i32, _vp, _vp, _i32, _i64, _i64, _vp, _i32, _i64, _vp]),
     "fm_grouped_gemm_ragged_k": (_i32, [_i32, _OPND, _OPND, _vp, _i32, _i64, _i64, _vp, _i32, _vp,
                                         _i64, _vp, _i64, _i64, _i32, _i64, _vp]),

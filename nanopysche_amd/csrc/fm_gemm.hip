@@ -1197,10 +1197,26 @@ __device__ __forceinline__ void store_bf16_passes(const v16f (&acc)[4][2], uint8
   else store_bf16_passes_v<false>(acc, W, C, ldC, row0, col0, w);
 }
 
+// K slices of each tile when the launch has fewer tiles than half of its
+// workgroups: an XCD's workgroups over its tiles, at least 16 steps a slice.
+// One tile alone takes 1.5 to 1.9 us a step (its loads, one step in flight, wait
+// for memory: weights of experts with few tokens are read once), and the idle
+// CUs take the other slices.
+__device__ __forceinline__ int ragged_m_slices(const TileQueue& q, int nk) {
+  const int by_cu = q.per_xcd > 0 ? q.nbx / q.per_xcd : 1, by_k = nk / 16;
+  const int s = by_cu < by_k ? by_cu : by_k;
+  return __builtin_amdgcn_readfirstlane(s < 1 ? 1 : s > 8 ? 8 : s);
+}
+// A slice's fp32 partial of a tile in the workspace: 256 KiB, wave by wave, 32
+// rows of 64 lanes x 16 bytes (4 consecutive columns i of the row j of the lane).
+constexpr int64_t kSliceFloats = 65536;
+
 // QNN (BF16 and FP8 pow2): the weight operand Q is stored [K][N]
 // (make_stream_nn16 / read_frag16_nn, make_stream_nn / read_frag8_nn); all N
 // tiles are full (N % 256 == 0, checked by the launcher).
-template <int KIND, int MXL = 0, bool QNN = false>
+// SPLIT: a launch of few tiles cuts each in K slices (ragged_m_slices) whose
+// partials go to the workspace C2 and are summed by slice_sum_kernel.
+template <int KIND, int MXL = 0, bool QNN = false, bool SPLIT = false>
 __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
   using SM = Smem256<KIND>;
   constexpr int ES = KIND == GK_BF16 ? 2 : 1;
@@ -1227,16 +1243,29 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
   TileQueue tq;
   tile_queue_init(p, tq, reinterpret_cast<int*>(smem + 2 * SM::kStage + kSpare));
   block_barrier();   // the tile queue is in LDS
+  int64_t nk = p.K / KSTEP;   // >= 2 (launcher)
+  int64_t k0 = 0;             // first step of this workgroup's slice
+  int slices = 1, slice = 0;
+  if constexpr (SPLIT) {
+    slices = ragged_m_slices(tq, int(nk));
+    if (slices > 1) {   // one slice of one tile per workgroup
+      slice = __builtin_amdgcn_readfirstlane(tq.c0 / tq.per_xcd);
+      if (slice >= slices) return;
+      tq.c0 -= slice * tq.per_xcd;
+      const int n = int(nk);
+      k0 = __builtin_amdgcn_readfirstlane(n * slice / slices);
+      nk = __builtin_amdgcn_readfirstlane(n * (slice + 1) / slices) - k0;
+    }
+  }
   TileP cur;
   if (!tile_queue_get(tq, 0, cur)) return;
   TileStreams S = tile_streams<KIND, QNN>(p.Q, p.P, p.n_i, cur, w);
-  const int64_t nk = p.K / KSTEP;   // >= 2 (launcher)
   const uint32_t smem_lds = lds_addr(smem);
   uint8_t* const W = smem + 2 * SM::kStage + w.wave * 2048;
 
   Frag<KIND> f0, f1;
-  issue_step<KIND, QNN>(S.q, S.p, S.sc, 0, smem_lds, w.wave);
-  issue_step<KIND, QNN>(S.q, S.p, S.sc, KSTEP, smem_lds + SM::kStage, w.wave);
+  issue_step<KIND, QNN>(S.q, S.p, S.sc, k0 * KSTEP, smem_lds, w.wave);
+  issue_step<KIND, QNN>(S.q, S.p, S.sc, (k0 + 1) * KSTEP, smem_lds + SM::kStage, w.wave);
   FM_WAIT_VMCNT(KIND == GK_BF16 ? 8 : 9);
   block_barrier();
   read_half<KIND, QNN>(smem, 0, f0, w);
@@ -1270,7 +1299,7 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
       __builtin_amdgcn_sched_barrier(0);
       FM_WAIT_VMCNT(0);
       block_barrier();
-      issue_read_half0<KIND, QNN>(S.q, S.p, S.sc, kn * KSTEP, smem_lds + cur_off, w.wave, smem + nxt_off, f0, w);
+      issue_read_half0<KIND, QNN>(S.q, S.p, S.sc, (k0 + kn) * KSTEP, smem_lds + cur_off, w.wave, smem + nxt_off, f0, w);
       mma_half<KIND>(f1, acc);
       interleave_half<KIND, QNN>();
       __builtin_amdgcn_sched_barrier(0);
@@ -1294,7 +1323,23 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
       we.lane = fresh_lane();
       we.lrow = we.lane & 31;
       we.lhalf = we.lane >> 5;
-      if (!p.out_f32) {
+      if (SPLIT && slices > 1) {
+        const int64_t slot = int64_t(tq.xcd * tq.per_xcd + tq.c0) * slices + slice;
+        float* dst = static_cast<float*>(p.C2) + slot * kSliceFloats + w.wave * 8192 + we.lane * 4;
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              st_global(dst + q * 256, make_float4(
+                  acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]));
+            dst += 1024;
+            __builtin_amdgcn_sched_barrier(0);   // one address at a time: registers
+          }
+      } else if (SPLIT) {   // bf16, pitch a multiple of 8 (launcher)
+        store_bf16_passes_v<true>(acc, W, static_cast<uint16_t*>(p.C), p.ldC, jb, ib, we);
+      } else if (!p.out_f32) {
         store_bf16_passes(acc, W, static_cast<uint16_t*>(p.C), p.ldC, jb, ib, we);
       } else {
         float* dst = static_cast<float*>(p.C) + jb * p.ldC + ib + we.lrow * p.ldC + 4 * we.lhalf;
@@ -1312,6 +1357,60 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
     cur = nxt;
   }
   FM_WAIT_VMCNT(0);  // no LDS-DMA may still be in flight when the workgroup exits
+}
+
+// Sums the slices of gemm256p_kernel<.., SPLIT> in slice order and writes the
+// bf16 rows: workgroup b the part of wave b % 8 of tile b / 8.  `nbx`: that
+// launch's workgroups per XCD.  Nothing to do when the tiles were not sliced.
+__global__ __launch_bounds__(256) void slice_sum_kernel(GemmParams p, int nk, int nbx) {
+  __shared__ __attribute__((aligned(16))) uint8_t W[16384];
+  __shared__ int qlds[256];
+  TileQueue tq;
+  tile_queue_init(p, tq, qlds);
+  tq.nbx = nbx;
+  const int slices = ragged_m_slices(tq, nk);
+  const int tile = int(blockIdx.x >> 3), wave = int(blockIdx.x & 7);
+  if (slices == 1 || tile >= tq.n_valid) return;
+  __syncthreads();
+  tq.xcd = tile / tq.per_xcd;
+  tq.c0 = tile - tq.xcd * tq.per_xcd;
+  TileP t;
+  if (!tile_queue_get(tq, 0, t)) return;
+  const int64_t ib = t.i0 + (wave >> 2) * 128, jb = t.j0 + (wave & 3) * 64;
+  if (ib >= p.n_i || jb >= t.j_end) return;
+  const int sub = threadIdx.x >> 6, lane = threadIdx.x & 63, lrow = lane & 31, lhalf = lane >> 5;
+  const float* src = static_cast<const float*>(p.C2) + int64_t(tile) * slices * kSliceFloats + wave * 8192 +
+                     sub * 2048 + lane * 4;
+  float4 v[8];
+#pragma unroll
+  for (int n = 0; n < 8; ++n) v[n] = *reinterpret_cast<const float4*>(src + n * 256);
+  for (int s = 1; s < slices; ++s) {
+    float4 u[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n) u[n] = *reinterpret_cast<const float4*>(src + s * kSliceFloats + n * 256);
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      v[n].x += u[n].x;
+      v[n].y += u[n].y;
+      v[n].z += u[n].z;
+      v[n].w += u[n].w;
+    }
+  }
+  // `sub` is the column block a; through LDS into whole 256-byte row segments
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    const int jr = (n >> 2) * 32 + lrow, q = n & 3;
+    *reinterpret_cast<uint2*>(W + jr * 256 + (((sub * 4 + q) ^ (jr & 15)) << 4) + lhalf * 8) =
+        make_uint2(hw_bf16x2(v[n].x, v[n].y), hw_bf16x2(v[n].z, v[n].w));
+  }
+  __syncthreads();
+  const int c = lane & 15;
+  uint16_t* const dst = static_cast<uint16_t*>(p.C) + jb * p.ldC + ib + c * 8;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int rr = sub * 16 + n * 4 + (lane >> 4);
+    st_global(dst + rr * p.ldC, *reinterpret_cast<const uint4*>(W + rr * 256 + ((c ^ (rr & 15)) << 4)));
+  }
 }
 
 // ============================================================================
@@ -2955,6 +3054,35 @@ int fm_grouped_gemm_ragged_m(int kind, const FmGemmOperand* tokens, const FmGemm
     return rc;
   if (p.m_tiles == 0) return 0;
   return dispatch_gemm<GM_RAGGED_M>(kind, p, static_cast<hipStream_t>(stream));
+}
+
+int fm_grouped_gemm_ragged_m_split(int kind, const FmGemmOperand* tokens, const FmGemmOperand* weights,
+                                   int64_t m_tiles, const int32_t* tile_expert, const int32_t* offsets, int E,
+                                   int64_t N, int64_t K, const int32_t* expert_mask, int mask_want, void* out,
+                                   int64_t ld_out, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int nn = (kind & FM_GEMM_W_KMAJOR) != 0;
+  kind &= ~FM_GEMM_W_KMAJOR;
+  GemmParams p;
+  if (int rc = ragged_m_params(kind, nn, 0, tokens, weights, m_tiles, tile_expert, offsets, E, N, K, expert_mask,
+                               mask_want, out, FM_DTYPE_BF16, ld_out, p))
+    return rc;
+  int64_t slots = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
+  if (workspace_bytes / (8 * kSliceFloats * 4) < slots) slots = workspace_bytes / (8 * kSliceFloats * 4);
+  FM_REQUIRE(kind == GK_BF16 && E <= 64 && K >= 128 && ld_out % 8 == 0 && (size_t(out) & 15) == 0,
+             "fm_grouped_gemm_ragged_m_split: BF16, E <= 64, K >= 128, a 16-byte aligned output and pitch");
+  FM_REQUIRE(workspace != nullptr && (size_t(workspace) & 15) == 0 && slots >= 1,
+             "fm_grouped_gemm_ragged_m_split: a 16-byte aligned workspace of 2 MiB or more");
+  if (p.m_tiles == 0) return 0;
+  if (int rc = prepare_gemm<GM_RAGGED_M>(kind, p)) return rc;
+  p.C2 = workspace;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid(unsigned(slots * 8)), block(512);
+  if (nn) hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, true, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, false, true>), grid, block, 0, s, p);
+  if (int rc = check_launch("fm_grouped_gemm_ragged_m_split")) return rc;
+  // two slices or more: at most half as many tiles as workgroups
+  hipLaunchKernelGGL(slice_sum_kernel, dim3(unsigned(slots * 4 * 8)), dim3(256), 0, s, p, int(K / 64), int(slots));
+  return check_launch("fm_grouped_gemm_ragged_m_split");
 }
 
 namespace {

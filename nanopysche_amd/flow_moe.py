@@ -572,6 +572,13 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
             gk |= _lib.GEMM_PAIRED | (_lib.GEMM_W_PAIRED if w.kmajor and w.paired else 0)
         elif w.paired:
             raise ValueError("paired-row weights need paired-row tokens")
+        if kind == _lib.QUANT_BF16 and _m_split(plan, w, out, mask):
+            ws = torch.empty(_cus(out.device) * _SLICE_BYTES, dtype=torch.uint8, device=out.device)
+            _lib.call("fm_grouped_gemm_ragged_m_split", gk, _token_operand(tokens, kind), w.operand(), plan.m_tiles,
+                      _lib.addr(plan.tile_expert), _lib.addr(plan.offsets), plan.num_experts, w.N, w.K,
+                      _lib.addr(mask), want, _lib.addr(out), out.stride(0), _lib.addr(ws), ws.numel(),
+                      _lib.stream_of(out))
+            return
         _lib.call("fm_grouped_gemm_ragged_m", gk, _token_operand(tokens, kind),
                   w.operand(), plan.m_tiles, _lib.addr(plan.tile_expert), _lib.addr(plan.offsets),
                   plan.num_experts, w.N, w.K,
@@ -581,6 +588,32 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
         launch()
     else:
         _timed(f"grouped_gemm_ragged_m/{_KIND_NAME[kind]}", 2.0 * _assignments(plan, mask, want) * w.N * w.K, launch)
+
+
+# A slice's fp32 partial of a 256 x 256 tile (fm_grouped_gemm_ragged_m_split).
+_SLICE_BYTES = 256 << 10
+_SPLIT_MIN_K = 4096
+
+
+def _m_split(plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool:
+    """A BF16 ragged-M launch that may leave half of the CUs without a tile (by
+    the assignments and, on average, half a tile per expert; any launch under
+    an expert mask) and whose K is long enough for the partials' round trip:
+    the device then slices K.  Measured unsliced against sliced, [K][N] weights:
+    8 experts of K 5632, N 2048, at 256 / 1024 / 2048 / 3072 tokens 128 / 139 /
+    141 / 136 us against 61 / 70 / 98 / 104; 8 of K 14336, N 4096, at 1024 394
+    against 268; 4 of K 4096, N 2048, at 512 / 1536 / 2048 / 3072 70 / 71 / 72 /
+    74 against 38 / 57 / 62 / 80, hence ``least``."""
+    if (w.K < _SPLIT_MIN_K or plan.num_experts > 64 or out.dtype != torch.bfloat16 or out.stride(0) % 8
+            or out.data_ptr() % 16):
+        return False
+    cus, ni = _cus(out.device), -(-w.N // 256)
+    if mask is not None:
+        return plan.m_tiles * ni <= 8 * cus
+    A, E = plan.num_tokens * plan.top_k, plan.num_experts
+    # two slices of a shorter K pay only where an expert's weights are read by few tiles
+    least = 2 if w.K >= 5632 or A <= 512 * E else 3
+    return least * ni * (A + 128 * E) <= 256 * cus
 
 
 # Model of a ragged-K launch for choosing its K split: ~1.3 us per 128-deep K
