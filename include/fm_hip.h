@@ -539,12 +539,13 @@ int fm_grouped_gemm_ragged_k(int kind, const FmGemmOperand* a_t, const FmGemmOpe
                              void* out2, int64_t out2_gs, int64_t split_rows, int out_dtype,
                              int64_t ld_out, void* stream);
 
-/* fm_grouped_gemm_ragged_m for BF16 weights of long K (FM_GEMM_W_KMAJOR or not,
- * bf16 output) when the tiles may be fewer than half of the CUs: the device then
- * cuts each tile in slices of K whose fp32 partials go to `workspace` (256 KiB a
- * workgroup, one workgroup per CU or as many as fit, at least 8; 16-byte
- * aligned) and sums them in slice order.  With more tiles the result and the
- * time are fm_grouped_gemm_ragged_m's. */
+/* fm_grouped_gemm_ragged_m for BF16 or paired FP8 operands (the kind's flags as
+ * there; bf16 output, 16-byte aligned, pitch a multiple of 8) when the tiles may
+ * be fewer than half of the CUs: the device then cuts each tile in slices of K
+ * whose fp32 partials go to `workspace` (256 KiB a workgroup, one workgroup per
+ * CU or as many as fit, at least 8; 16-byte aligned) and sums them in slice
+ * order.  With more tiles, or a short K, the result is
+ * fm_grouped_gemm_ragged_m's. */
 int fm_grouped_gemm_ragged_m_split(int kind, const FmGemmOperand* tokens, const FmGemmOperand* weights,
                                    int64_t m_tiles, const int32_t* tile_expert, const int32_t* offsets, int E,
                                    int64_t N, int64_t K, const int32_t* expert_mask, int mask_want, void* out,

@@ -1197,19 +1197,43 @@ __device__ __forceinline__ void store_bf16_passes(const v16f (&acc)[4][2], uint8
   else store_bf16_passes_v<false>(acc, W, C, ldC, row0, col0, w);
 }
 
-// K slices of each tile when the launch has fewer tiles than half of its
-// workgroups: an XCD's workgroups over its tiles, at least 16 steps a slice.
-// One tile alone takes 1.5 to 1.9 us a step (its loads, one step in flight, wait
-// for memory: weights of experts with few tokens are read once), and the idle
-// CUs take the other slices.
-__device__ __forceinline__ int ragged_m_slices(const TileQueue& q, int nk) {
-  const int by_cu = q.per_xcd > 0 ? q.nbx / q.per_xcd : 1, by_k = nk / 16;
-  const int s = by_cu < by_k ? by_cu : by_k;
-  return __builtin_amdgcn_readfirstlane(s < 1 ? 1 : s > 8 ? 8 : s);
+// K slices of each tile when the launch has at most half as many tiles as
+// workgroups.  One tile alone takes 1.1 to 1.9 us a step (its loads, a step or
+// two in flight, wait for memory: weights of experts with few tokens are read
+// once), and the idle CUs take the other slices.  The time of s slices in steps:
+// nk / s, a launch, and the partials' way out and back, 0.1 us a slice and tile
+// (a step as 1.4 us for BF16, 1.15 us for FP8).  At least 8 steps a slice.
+constexpr int kSliceSteps = 8, kMaxSlices = 8;
+__device__ __forceinline__ int ragged_m_slices(const TileQueue& q, int nk, bool bf16) {
+  const int by_cu = q.per_xcd > 0 ? q.nbx / q.per_xcd : 1, by_k = nk / kSliceSteps;
+  const float launch = bf16 ? 5.f : 6.5f, part = float(q.n_valid) * (bf16 ? 1.f / 14 : 1.f / 11);
+  int best = 1;
+  float cost = float(nk);
+  for (int s = 2; s <= kMaxSlices && s <= by_cu && s <= by_k; ++s) {
+    const float c = float(nk) / float(s) + launch + part * float(s);
+    if (c < cost) {
+      cost = c;
+      best = s;
+    }
+  }
+  return __builtin_amdgcn_readfirstlane(best);
 }
 // A slice's fp32 partial of a tile in the workspace: 256 KiB, wave by wave, 32
 // rows of 64 lanes x 16 bytes (4 consecutive columns i of the row j of the lane).
 constexpr int64_t kSliceFloats = 65536;
+__device__ __forceinline__ void store_slice(float* dst, const v16f (&acc)[4][2]) {
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        st_global(dst + q * 256, make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2],
+                                             acc[a][b][4 * q + 3]));
+      dst += 1024;
+      __builtin_amdgcn_sched_barrier(0);   // one address at a time: registers
+    }
+}
 
 // QNN (BF16 and FP8 pow2): the weight operand Q is stored [K][N]
 // (make_stream_nn16 / read_frag16_nn, make_stream_nn / read_frag8_nn); all N
@@ -1247,7 +1271,7 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
   int64_t k0 = 0;             // first step of this workgroup's slice
   int slices = 1, slice = 0;
   if constexpr (SPLIT) {
-    slices = ragged_m_slices(tq, int(nk));
+    slices = ragged_m_slices(tq, int(nk), KIND == GK_BF16);
     if (slices > 1) {   // one slice of one tile per workgroup
       slice = __builtin_amdgcn_readfirstlane(tq.c0 / tq.per_xcd);
       if (slice >= slices) return;
@@ -1325,18 +1349,7 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
       we.lhalf = we.lane >> 5;
       if (SPLIT && slices > 1) {
         const int64_t slot = int64_t(tq.xcd * tq.per_xcd + tq.c0) * slices + slice;
-        float* dst = static_cast<float*>(p.C2) + slot * kSliceFloats + w.wave * 8192 + we.lane * 4;
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              st_global(dst + q * 256, make_float4(
-                  acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]));
-            dst += 1024;
-            __builtin_amdgcn_sched_barrier(0);   // one address at a time: registers
-          }
+        store_slice(static_cast<float*>(p.C2) + slot * kSliceFloats + w.wave * 8192 + we.lane * 4, acc);
       } else if (SPLIT) {   // bf16, pitch a multiple of 8 (launcher)
         store_bf16_passes_v<true>(acc, W, static_cast<uint16_t*>(p.C), p.ldC, jb, ib, we);
       } else if (!p.out_f32) {
@@ -1359,16 +1372,16 @@ __global__ __launch_bounds__(512) void gemm256p_kernel(GemmParams p) {
   FM_WAIT_VMCNT(0);  // no LDS-DMA may still be in flight when the workgroup exits
 }
 
-// Sums the slices of gemm256p_kernel<.., SPLIT> in slice order and writes the
-// bf16 rows: workgroup b the part of wave b % 8 of tile b / 8.  `nbx`: that
+// Sums the slices of gemm256p_kernel / gemm256r_kernel <.., SPLIT> in slice order
+// and writes the bf16 rows: workgroup b the part of wave b % 8 of tile b / 8.  `nbx`: that
 // launch's workgroups per XCD.  Nothing to do when the tiles were not sliced.
-__global__ __launch_bounds__(256) void slice_sum_kernel(GemmParams p, int nk, int nbx) {
+__global__ __launch_bounds__(256) void slice_sum_kernel(GemmParams p, int nk, int nbx, bool bf16) {
   __shared__ __attribute__((aligned(16))) uint8_t W[16384];
   __shared__ int qlds[256];
   TileQueue tq;
   tile_queue_init(p, tq, qlds);
   tq.nbx = nbx;
-  const int slices = ragged_m_slices(tq, nk);
+  const int slices = ragged_m_slices(tq, nk, bf16);
   const int tile = int(blockIdx.x >> 3), wave = int(blockIdx.x & 7);
   if (slices == 1 || tile >= tq.n_valid) return;
   __syncthreads();
@@ -2118,8 +2131,10 @@ __device__ __forceinline__ bool rk_next_min(const RkQueue& q, int& c, TileK& t, 
 // last four refills of a tile fetch the next tile's first four halves;
 // ragged-K tiles of one K step come last, one at a time.  No
 // expert masks, at most 64 experts, ragged-M K >= 384 (the launcher).
-template <int KIND, int MXL, bool HAS_M, bool HAS_K, bool QNN, bool QP>
+// SPLIT (HAS_M alone): as gemm256p_kernel's, in whole steps of two halves.
+template <int KIND, int MXL, bool HAS_M, bool HAS_K, bool QNN, bool QP, bool SPLIT = false>
 __global__ __launch_bounds__(512) void gemm256r_kernel(GemmParams pm, GemmParams pk) {
+  static_assert(!SPLIT || (HAS_M && !HAS_K), "slices of ragged-M tiles");
   static_assert(!(HAS_K && QNN), "ragged-K tiles share the NT fragment reads");
   static_assert(KIND == GK_FP8_POW2 || (KIND == GK_FP8_MX && !QNN), "pow2, or MX with [N][K] weights");
   using SM = SmemR<KIND>;
@@ -2191,12 +2206,23 @@ __global__ __launch_bounds__(512) void gemm256r_kernel(GemmParams pm, GemmParams
 
   const int nh_m = HAS_M ? int(pm.K / 64) : 0;   // >= 6 (launcher)
   int cm = 0, ck = 0;                              // positions in the two shares
+  int slices = 1, slice = 0, kh0 = 0, nh = nh_m;   // this workgroup's halves of each tile
+  if constexpr (SPLIT) {
+    slices = ragged_m_slices(tq, nh_m / 2, false);
+    if (slices > 1) {   // one slice of one tile per workgroup
+      slice = __builtin_amdgcn_readfirstlane(tq.c0 / tq.per_xcd);
+      if (slice >= slices) return;
+      tq.c0 -= slice * tq.per_xcd;
+      kh0 = __builtin_amdgcn_readfirstlane((nh_m / 2) * slice / slices * 2);
+      nh = __builtin_amdgcn_readfirstlane((nh_m / 2) * (slice + 1) / slices * 2) - kh0;
+    }
+  }
   auto next_item = [&](ItemR& it) -> bool {
     if constexpr (HAS_M) {
       TileP tp;
       if (tile_queue_get(tq, cm, tp)) {
         ++cm;
-        it = ItemR{0, tp.e, tp.i0, tp.j0, tp.j_end, 0, nh_m};
+        it = ItemR{0, tp.e, tp.i0, tp.j0, tp.j_end, SPLIT ? kh0 : 0, SPLIT ? nh : nh_m};
         return true;
       }
     }
@@ -2260,6 +2286,19 @@ __global__ __launch_bounds__(512) void gemm256r_kernel(GemmParams pm, GemmParams
     } else {   // dgrad / forward: row j (token), column i
       const int p_rows = it.j_end - it.j0 < kT ? it.j_end - it.j0 : kT;
       if (ib >= rfl64(plm->n_i) || jb >= it.j0 + p_rows) return 0;
+      if (SPLIT && slices > 1) {
+        const int64_t slot = int64_t(tq.xcd * tq.per_xcd + tq.c0) * slices + slice;
+        store_slice(static_cast<float*>(plm->C2) + slot * kSliceFloats + w.wave * 8192 + fresh_lane() * 4, acc);
+        return 0;   // the workgroup's only tile
+      }
+      if constexpr (SPLIT) {   // bf16, pitch a multiple of 8 (launcher)
+        WaveCoord we = w;
+        we.lane = fresh_lane();
+        we.lrow = we.lane & 31;
+        we.lhalf = we.lane >> 5;
+        store_bf16_passes_v<true>(acc, W, static_cast<uint16_t*>(plm->C), rfl64(plm->ldC), jb, ib, we);
+        return 16;
+      }
       return store(plm->C, rfl64(plm->ldC), __builtin_amdgcn_readfirstlane(plm->out_f32), jb, ib, acc);
     }
   };
@@ -3061,15 +3100,19 @@ int fm_grouped_gemm_ragged_m_split(int kind, const FmGemmOperand* tokens, const 
                                    int64_t N, int64_t K, const int32_t* expert_mask, int mask_want, void* out,
                                    int64_t ld_out, void* workspace, int64_t workspace_bytes, void* stream) {
   const int nn = (kind & FM_GEMM_W_KMAJOR) != 0;
-  kind &= ~FM_GEMM_W_KMAJOR;
+  const int paired = (kind & FM_GEMM_PAIRED) == 0 ? 0 : (nn && (kind & FM_GEMM_W_PAIRED) != 0) ? 2 : 1;
+  FM_REQUIRE((kind & FM_GEMM_W_PAIRED) == 0 || (nn && paired),
+             "fm_grouped_gemm_ragged_m_split: FM_GEMM_W_PAIRED needs FM_GEMM_PAIRED and FM_GEMM_W_KMAJOR");
+  kind &= ~(FM_GEMM_W_KMAJOR | FM_GEMM_PAIRED | FM_GEMM_W_PAIRED);
   GemmParams p;
-  if (int rc = ragged_m_params(kind, nn, 0, tokens, weights, m_tiles, tile_expert, offsets, E, N, K, expert_mask,
+  if (int rc = ragged_m_params(kind, nn, paired, tokens, weights, m_tiles, tile_expert, offsets, E, N, K, expert_mask,
                                mask_want, out, FM_DTYPE_BF16, ld_out, p))
     return rc;
   int64_t slots = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
   if (workspace_bytes / (8 * kSliceFloats * 4) < slots) slots = workspace_bytes / (8 * kSliceFloats * 4);
-  FM_REQUIRE(kind == GK_BF16 && E <= 64 && K >= 128 && ld_out % 8 == 0 && (size_t(out) & 15) == 0,
-             "fm_grouped_gemm_ragged_m_split: BF16, E <= 64, K >= 128, a 16-byte aligned output and pitch");
+  FM_REQUIRE((kind == GK_BF16 || paired) && E <= 64 && K >= 128 && ld_out % 8 == 0 && (size_t(out) & 15) == 0,
+             "fm_grouped_gemm_ragged_m_split: BF16 or paired operands, E <= 64, K >= 128, a 16-byte aligned output "
+             "and pitch");
   FM_REQUIRE(workspace != nullptr && (size_t(workspace) & 15) == 0 && slots >= 1,
              "fm_grouped_gemm_ragged_m_split: a 16-byte aligned workspace of 2 MiB or more");
   if (p.m_tiles == 0) return 0;
@@ -3077,11 +3120,27 @@ int fm_grouped_gemm_ragged_m_split(int kind, const FmGemmOperand* tokens, const 
   p.C2 = workspace;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid(unsigned(slots * 8)), block(512);
-  if (nn) hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, true, true>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, false, true>), grid, block, 0, s, p);
+  if (kind == GK_BF16) {
+    if (nn) hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, true, true>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm256p_kernel<GK_BF16, 0, false, true>), grid, block, 0, s, p);
+  } else if (kind == GK_FP8_POW2) {
+    if (paired == 2)
+      hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_POW2, 0, true, false, true, true, true>), grid, block, 0, s, p, p);
+    else if (nn)
+      hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_POW2, 0, true, false, true, false, true>), grid, block, 0, s, p, p);
+    else hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_POW2, 0, true, false, false, true, true>), grid, block, 0, s, p, p);
+  } else {
+    switch ((p.Q.s_kb != 1 ? 1 : 0) | (p.P.s_kb != 1 ? 2 : 0)) {
+      case 0: hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_MX, 0, true, false, false, true, true>), grid, block, 0, s, p, p); break;
+      case 1: hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_MX, 1, true, false, false, true, true>), grid, block, 0, s, p, p); break;
+      case 2: hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_MX, 2, true, false, false, true, true>), grid, block, 0, s, p, p); break;
+      default: hipLaunchKernelGGL((gemm256r_kernel<GK_FP8_MX, 3, true, false, false, true, true>), grid, block, 0, s, p, p); break;
+    }
+  }
   if (int rc = check_launch("fm_grouped_gemm_ragged_m_split")) return rc;
   // two slices or more: at most half as many tiles as workgroups
-  hipLaunchKernelGGL(slice_sum_kernel, dim3(unsigned(slots * 4 * 8)), dim3(256), 0, s, p, int(K / 64), int(slots));
+  hipLaunchKernelGGL(slice_sum_kernel, dim3(unsigned(slots * 4 * 8)), dim3(256), 0, s, p,
+                     int(K / (kind == GK_BF16 ? 64 : 128)), int(slots), kind == GK_BF16);
   return check_launch("fm_grouped_gemm_ragged_m_split");
 }
 

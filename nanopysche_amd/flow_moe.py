@@ -572,7 +572,7 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
             gk |= _lib.GEMM_PAIRED | (_lib.GEMM_W_PAIRED if w.kmajor and w.paired else 0)
         elif w.paired:
             raise ValueError("paired-row weights need paired-row tokens")
-        if kind == _lib.QUANT_BF16 and _m_split(plan, w, out, mask):
+        if (t_paired or kind == _lib.QUANT_BF16) and _m_split(kind, plan, w, out, mask):
             ws = torch.empty(_cus(out.device) * _SLICE_BYTES, dtype=torch.uint8, device=out.device)
             _lib.call("fm_grouped_gemm_ragged_m_split", gk, _token_operand(tokens, kind), w.operand(), plan.m_tiles,
                       _lib.addr(plan.tile_expert), _lib.addr(plan.offsets), plan.num_experts, w.N, w.K,
@@ -592,28 +592,34 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
 
 # A slice's fp32 partial of a 256 x 256 tile (fm_grouped_gemm_ragged_m_split).
 _SLICE_BYTES = 256 << 10
-_SPLIT_MIN_K = 4096
+_SLICE_GAIN = 5.25   # K steps (about 6 us) that slicing must save by the model
 
 
-def _m_split(plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool:
-    """A BF16 ragged-M launch that may leave half of the CUs without a tile (by
-    the assignments and, on average, half a tile per expert; any launch under
-    an expert mask) and whose K is long enough for the partials' round trip:
-    the device then slices K.  Measured unsliced against sliced, [K][N] weights:
-    8 experts of K 5632, N 2048, at 256 / 1024 / 2048 / 3072 tokens 128 / 139 /
-    141 / 136 us against 61 / 70 / 98 / 104; 8 of K 14336, N 4096, at 1024 394
-    against 268; 4 of K 4096, N 2048, at 512 / 1536 / 2048 / 3072 70 / 71 / 72 /
-    74 against 38 / 57 / 62 / 80, hence ``least``."""
-    if (w.K < _SPLIT_MIN_K or plan.num_experts > 64 or out.dtype != torch.bfloat16 or out.stride(0) % 8
-            or out.data_ptr() % 16):
-        return False
+def _m_split(kind, plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool:
+    """A ragged-M launch (BF16, or paired FP8) that is expected to leave at
+    least half of the CUs without a tile and whose K is long enough for the
+    partials' round trip: the device then slices K by the tiles that there are
+    (ragged_m_slices, whose costs these are).  Under an expert mask the tiles
+    are not known: any BF16 launch (its experts are those with few tokens) of 64
+    steps.  Measured unsliced against sliced, [K][N] weights, tokens over all
+    experts 512 / 1024 / 2048: BF16, 8 experts of K 5632, N 2048, 128 / 139 /
+    140 us against 59 / 70 / 99; of K 2048 38 / 40 / 42 against 33 / 40 / 49 (not
+    sliced); 8 of K 14336, N 4096, at 512 / 1024 351 / 393 against 228 / 265; pow2
+    127 / 154 against 115 / 135.  More than 512 tokens an expert read a weight
+    tile often enough for steps as short as FP8's: 4 of K 4096, N 2048, at 3072
+    79 against 81 (not sliced)."""
+    E, bf16 = plan.num_experts, kind == _lib.QUANT_BF16
+    nk = w.K // (64 if bf16 else 128)
+    if nk < 20 or E > 64 or out.dtype != torch.bfloat16 or out.stride(0) % 8 or out.data_ptr() % 16:
+        return False   # (under 20 steps no slicing gains as much)
     cus, ni = _cus(out.device), -(-w.N // 256)
     if mask is not None:
-        return plan.m_tiles * ni <= 8 * cus
-    A, E = plan.num_tokens * plan.top_k, plan.num_experts
-    # two slices of a shorter K pay only where an expert's weights are read by few tiles
-    least = 2 if w.K >= 5632 or A <= 512 * E else 3
-    return least * ni * (A + 128 * E) <= 256 * cus
+        return bf16 and nk >= 64 and plan.m_tiles * ni <= 8 * cus
+    A = plan.num_tokens * plan.top_k
+    tiles = ni * E * max(1.0, A / E / 256 + 0.5)
+    launch, part = (5.0, tiles / 14) if bf16 and A <= 512 * E else (6.5, tiles / 11)
+    return any(nk / s + launch + part * s + _SLICE_GAIN <= nk
+               for s in range(2, 9) if s * tiles <= cus and 8 * s <= nk)
 
 
 # Model of a ragged-K launch for choosing its K split: ~1.3 us per 128-deep K

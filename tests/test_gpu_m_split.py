@@ -1,4 +1,4 @@
-"""BF16 ragged-M GEMM whose few tiles are cut in slices of K, against float64: bf16
+"""Ragged-M GEMM whose few tiles are cut in slices of K, against float64 (BF16): bf16
 products are exact in fp32, so a sum over K, in slices or not, is off by at most
 K 2^-24 sum |terms|, and the bf16 output by half a unit of its last place more."""
 
@@ -7,7 +7,7 @@ import torch
 
 import nanopysche_amd as fm
 from nanopysche_amd import _lib
-from nanopysche_amd.flow_moe import ExpertWeightOperand, _gemm_kind, _m_split, _token_operand
+from nanopysche_amd.flow_moe import ExpertWeightOperand, ExpertWeights, _gemm_kind, _m_split, _token_operand
 from tests.helpers import randn_bf16
 
 pytestmark = pytest.mark.gpu
@@ -55,8 +55,45 @@ def test_matches_float64(dev, counts, masked, K, groups, form):
     assert torch.all(out[offs[E]:] == 7.0)
 
 
+@pytest.mark.parametrize("kind,kmajor", [("pow2", False), ("pow2", True), ("mx", False)])
+@pytest.mark.parametrize("counts", [(300, 0, 1, 257), (130, 200)])
+def test_paired_matches_unsliced(dev, counts, kind, kmajor):
+    """FP8: the sliced sums against the same products in one sweep of K, both in
+    fp32: K 2^-23 sum |terms| apart at most, and a bf16 rounding each."""
+    E, K, N = len(counts), 6784, 512   # 53 steps: uneven slices
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int64) for e, c in enumerate(counts)])[:, None].to(dev)
+    plan = fm.route_tokens(idx, E)
+    pow2 = kind == "pow2"
+    k = _lib.QUANT_POW2 if pow2 else _lib.QUANT_MX
+    x = randn_bf16((sum(counts), K), seed=1).to(dev)
+    wd = randn_bf16((E * K, N), seed=2, std=0.1).to(dev)
+    ew = ExpertWeights(k, paired=True).refresh(wd, wd, wd, E, False)
+    pt = fm.fused_permute_pad(x, plan, E, granularity="1x128" if pow2 else "1x32", pow2_scale=pow2,
+                              kmajor_scales=kmajor, paired_rows=True)
+    w = ew.w2t
+    assert w.K == K and w.N == N
+    ws = torch.full((256 * 65536,), float("nan"), device=dev)
+    gk = _gemm_kind(k) | _lib.GEMM_PAIRED | (_lib.GEMM_W_KMAJOR if w.kmajor else 0) | (
+        _lib.GEMM_W_PAIRED if w.kmajor and w.paired else 0)
+    args = (gk, _token_operand(pt.rows, k), w.operand(), plan.m_tiles, _lib.addr(plan.tile_expert),
+            _lib.addr(plan.offsets), E, N, K, None, 1)
+    a, b = (torch.full((plan.rows_max, N), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    _lib.call("fm_grouped_gemm_ragged_m", *args, _lib.addr(a), _lib.DTYPE_BF16, N, _lib.stream_of(a))
+    _lib.call("fm_grouped_gemm_ragged_m_split", *args, _lib.addr(b), N, _lib.addr(ws), ws.numel() * 4,
+              _lib.stream_of(b))
+    assert not torch.isnan(ws).all()   # slices were made
+    offs = plan.offsets.tolist()
+    for e, c in enumerate(counts):
+        # quantisation moves a term by 1/8 of its size at most (e4m3, three mantissa bits, each factor 1/16)
+        xe = x[idx[:, 0] == e].abs().double()
+        terms = 1.25 * (xe @ wd[e * K:(e + 1) * K].abs().double())
+        g, h = a[offs[e]:offs[e] + c].double(), b[offs[e]:offs[e] + c].double()
+        assert torch.all((g - h).abs() <= K * 2.0 ** -23 * terms + 2.0 ** -8 * (g.abs() + h.abs()))
+    assert torch.all(b[offs[E]:] == 7.0)
+
+
 def test_rule(dev):
-    """Few tiles of a long K, by the host's bound; any launch under a mask."""
+    """Few tiles of a long K, by the host's bound; BF16 of 64 steps under a mask."""
     def w(N, K):
         return ExpertWeightOperand(None, None, K, N * K, N=N, K=K)
 
@@ -66,9 +103,14 @@ def test_rule(dev):
     def out(N):
         return torch.empty(256, N, dtype=torch.bfloat16, device=dev)
 
+    bf, p2 = _lib.QUANT_BF16, _lib.QUANT_POW2
     some = torch.ones(4, dtype=torch.int32, device=dev)
-    assert _m_split(plan(1024), w(2048, 4096), out(2048), None)
-    assert not _m_split(plan(1024), w(2048, 3968), out(2048), None)
-    assert not _m_split(plan(8192), w(2048, 4096), out(2048), None)
-    assert _m_split(plan(8192), w(2048, 4096), out(2048), some)
-    assert not _m_split(plan(1024), w(2048, 4096), out(2048).float(), None)
+    assert _m_split(bf, plan(1024), w(2048, 4096), out(2048), None)
+    assert not _m_split(bf, plan(1024), w(2048, 1024), out(2048), None)
+    assert not _m_split(bf, plan(3072), w(2048, 4096), out(2048), None)
+    assert not _m_split(bf, plan(8192), w(2048, 14336), out(2048), None)
+    assert not _m_split(bf, plan(1024), w(2048, 4096), out(2048).float(), None)
+    assert _m_split(p2, plan(512), w(1024, 4096), out(1024), None)
+    assert not _m_split(p2, plan(2048), w(2048, 4096), out(2048), None)
+    assert _m_split(bf, plan(8192), w(2048, 4096), out(2048), some)
+    assert not _m_split(p2, plan(8192), w(2048, 14336), out(2048), some)
