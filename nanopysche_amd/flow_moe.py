@@ -601,7 +601,9 @@ def _m_split(kind, plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool
     partials' round trip: the device then slices K by the tiles that there are
     (ragged_m_slices, whose costs these are).  Under an expert mask the tiles
     are not known: any BF16 launch (its experts are those with few tokens) of 64
-    steps.  Measured unsliced against sliced, [K][N] weights, tokens over all
+    steps, or 88 with more than 512 tokens an expert (steps of half of 8 experts of
+    2048 x 5632 in BF16, 2048 / 8192 tokens, 1566 / 2960 us against 1291 / 2850; 16
+    of 1024 x 4096 with 1024 each 1890 against 1902 with 64 for all).  Measured unsliced against sliced, [K][N] weights, tokens over all
     experts 512 / 1024 / 2048: BF16, 8 experts of K 5632, N 2048, 128 / 139 /
     140 us against 59 / 70 / 99; of K 2048 38 / 40 / 42 against 33 / 40 / 49 (not
     sliced); 8 of K 14336, N 4096, at 512 / 1024 351 / 393 against 228 / 265; pow2
@@ -613,9 +615,9 @@ def _m_split(kind, plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool
     if nk < 20 or E > 64 or out.dtype != torch.bfloat16 or out.stride(0) % 8 or out.data_ptr() % 16:
         return False   # (under 20 steps no slicing gains as much)
     cus, ni = _cus(out.device), -(-w.N // 256)
-    if mask is not None:
-        return bf16 and nk >= 64 and plan.m_tiles * ni <= 8 * cus
     A = plan.num_tokens * plan.top_k
+    if mask is not None:
+        return bf16 and nk >= (64 if A <= 512 * E else 88) and plan.m_tiles * ni <= 8 * cus
     tiles = ni * E * max(1.0, A / E / 256 + 0.5)
     launch, part = (5.0, tiles / 14) if bf16 and A <= 512 * E else (6.5, tiles / 11)
     return any(nk / s + launch + part * s + _SLICE_GAIN <= nk

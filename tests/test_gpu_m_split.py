@@ -93,7 +93,7 @@ def test_paired_matches_unsliced(dev, counts, kind, kmajor):
 
 
 def test_rule(dev):
-    """Few tiles of a long K, by the host's bound; BF16 of 64 steps under a mask."""
+    """Few tiles of a long K, by the host's bound; BF16 of 64 or 88 steps under a mask."""
     def w(N, K):
         return ExpertWeightOperand(None, None, K, N * K, N=N, K=K)
 
@@ -112,5 +112,7 @@ def test_rule(dev):
     assert not _m_split(bf, plan(1024), w(2048, 4096), out(2048).float(), None)
     assert _m_split(p2, plan(512), w(1024, 4096), out(1024), None)
     assert not _m_split(p2, plan(2048), w(2048, 4096), out(2048), None)
-    assert _m_split(bf, plan(8192), w(2048, 4096), out(2048), some)
+    assert _m_split(bf, plan(8192), w(2048, 5632), out(2048), some)
+    assert not _m_split(bf, plan(8192), w(2048, 4096), out(2048), some)
+    assert _m_split(bf, plan(2048), w(2048, 4096), out(2048), some)
     assert not _m_split(p2, plan(8192), w(2048, 14336), out(2048), some)
