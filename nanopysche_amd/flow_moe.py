@@ -1183,6 +1183,12 @@ class FP8FlowMoECompute:
         T, D = x.shape
         E, H = self.num_experts, self.hidden_size
         K = indices.shape[1]
+        # before any launch: the plan's assignments index x's rows, and the
+        # unpermute reads a weight per assignment
+        if indices.shape[0] != T:
+            raise ValueError(f"indices are for {indices.shape[0]} tokens, x has {T}")
+        if weights.shape[0] < T:
+            raise ValueError(f"weights are for {weights.shape[0]} tokens, x has {T}")
         fp8_kind, use_bf16 = self.modes(T * K)
         dev = x.device
         thr = self.fp8_gemm_threshold if fp8_kind is not None else 1 << 62
