@@ -221,7 +221,10 @@ def require_device(t: torch.Tensor, name: str = "tensor") -> None:
 def stream_of(t: torch.Tensor) -> int:
     """The handle of the current stream of t's device (0.1 us; through a
     torch.cuda.Stream object it took 2.2 us, once per launch)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    index = t.get_device()
+    if index < 0:   # the raw call would take -1 as the current device
+        raise ValueError(f"expected a tensor on a ROCm device, got one on {t.device} (there is no CPU fallback)")
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t) -> C.c_void_p:
