@@ -360,9 +360,10 @@ __global__ __launch_bounds__(256) void gate_pieces_kernel(GatePieceArgs a) {
 // ---------------------------------------------------------------- dx ----
 // A wave forms 64 tokens x 64 columns (4 waves: 128 x 128, the shared fragments
 // from the L1), every fragment one coalesced read: K = Ep experts once per pair of pieces, the small pairs first, the
-// two high pieces last.  With an fp32 gate six of the nine pairs (down to
-// 2^-16 of the product; the rest are below its fp32 rounding).  A lane ends
-// with 16 consecutive columns of a token.
+// two high pieces last.  All nine pairs with an fp32 gate: the pieces are
+// truncations, so the three smallest pairs have the product's sign and come to
+// 2^-21 of it, more than an fp32 rounding.  A lane ends with 16 consecutive
+// columns of a token.
 struct GateDxArgs {
   const uint16_t* p;     // [3][Tp x Ep] fragments
   const uint16_t* wt;    // [1 or 3][Dp x Ep] fragments
@@ -386,9 +387,9 @@ __global__ __launch_bounds__(256) void gate_dx_kernel(GateDxArgs a) {
     wr[f] = a.wt + (d0 / 16 + f) * (16 * a.Ep) + 8 * lane;
   }
   const int64_t pp = a.Tp * a.Ep, wp = a.Dp * a.Ep;
-  constexpr int kPairs = W32 ? 6 : 3;
-  constexpr int kP[6] = {W32 ? 0 : 2, W32 ? 2 : 1, W32 ? 1 : 0, 0, 1, 0};   // dlogits piece
-  constexpr int kW[6] = {W32 ? 2 : 0, 0, W32 ? 1 : 0, 1, 0, 0};             // gate piece
+  constexpr int kPairs = W32 ? 9 : 3;
+  constexpr int kP[9] = {2, 1, W32 ? 2 : 0, 0, 2, 1, 0, 1, 0};   // dlogits piece
+  constexpr int kW[9] = {W32 ? 2 : 0, W32 ? 2 : 0, W32 ? 1 : 0, 2, 0, 1, 1, 0, 0};   // gate piece
   v4f acc[4][4];   // [column fragment][token fragment]
 #pragma unroll
   for (int f = 0; f < 4; ++f)

@@ -5,13 +5,13 @@ slices of tokens.
 
 Bounds: every product of pieces is exact in fp32, so a sum over n is off by at
 most (n + 2) 2^-24 sum |terms|, the 2 for the low pieces joining the high ones
-(n 2^-23 for the six pairs of pieces of two fp32 factors, which leave out
-terms below 2^-24 of a product)."""
+(n 2^-23 for the nine pairs of pieces of two fp32 factors)."""
 
 import pytest
 import torch
 
 import nanopysche_amd as fm
+from nanopysche_amd import _lib
 from nanopysche_amd.routing import router_backward, router_forward
 
 pytestmark = pytest.mark.gpu
@@ -60,6 +60,34 @@ def test_products_at_tile_edges(dev, T, D, E, gate):
     assert torch.all((db.double() - dl64.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * dl64.abs().sum(0) + 1e-30)
     only = router_backward(st, x, w, dws, daux, need_w=False, need_b=False)[0]
     assert torch.equal(only, dx)
+
+
+@pytest.mark.parametrize("T,D,E", [(40, 136, 9), (64, 264, 40), (64, 4104, 3)])
+def test_dx_of_fp32_factors_has_every_product(dev, T, D, E):
+    """dlogits a and gate b, all low mantissa bits set, in expert 0; the product's two
+    fp32 halves (a b = p + r exactly) against -1 in two other experts: dx[t, t] is 0.  The terms
+    stay below 2, so the sums (at most four of that size: the two high pieces and what is
+    carried) are off by 2^-22 at most, where the three smallest pairs of pieces alone are 2^-21."""
+    n = min(T, D)
+    k = torch.arange(n) % 32
+    a = 1 + k / 128 + 2.0 ** -7 - 2.0 ** -23
+    b = 1 + k.flip(0) / 128 + 2.0 ** -7 - 2.0 ** -23
+    a, b = a.float(), b.float()
+    prod = a.double() * b.double()
+    p = prod.float()
+    r = (prod - p.double()).float()
+    assert torch.equal(p.double() + r.double(), prod) and float(p.max()) < 2
+    dl, w = torch.zeros(T, E), torch.zeros(E, D)
+    dl[:n, 0], w[0, :n] = a, b
+    dl[:, 1] = dl[:, E - 1] = -1
+    w[1, :n], w[E - 1, :n] = p, r
+    dl, w, x = dl.to(dev), w.to(dev), torch.zeros(T, D, dtype=torch.bfloat16, device=dev)
+    dx = torch.empty_like(x)
+    ws = torch.empty(_lib.size_of("fm_router_workspace_bytes", T, D, E), dtype=torch.uint8, device=dev)
+    _lib.call("fm_router_backward", _lib.addr(dl), E, _lib.addr(x), _lib.DTYPE_BF16, D, T, D, _lib.addr(w),
+              _lib.DTYPE_F32, D, E, _lib.addr(dx), D, None, _lib.DTYPE_F32, 0, None, _lib.DTYPE_F32, _lib.addr(ws),
+              ws.numel(), _lib.stream_of(x))
+    assert float(dx.diagonal()[:n].abs().max()) <= 2.0 ** -22
 
 
 @pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
