@@ -44,6 +44,7 @@
 #include <cstdlib>
 
 #include "fm_common.h"
+#include "fm_slices.h"
 #include <type_traits>
 #include "../../include/fm_hip.h"
 
@@ -1198,25 +1199,10 @@ __device__ __forceinline__ void store_bf16_passes(const v16f (&acc)[4][2], uint8
 }
 
 // K slices of each tile when the launch has at most half as many tiles as
-// workgroups.  One tile alone takes 1.1 to 1.9 us a step (its loads, a step or
-// two in flight, wait for memory: weights of experts with few tokens are read
-// once), and the idle CUs take the other slices.  The time of s slices in steps:
-// nk / s, a launch, and the partials' way out and back, 0.1 us a slice and tile
-// (a step as 1.4 us for BF16, 1.15 us for FP8).  At least 8 steps a slice.
-constexpr int kSliceSteps = 8, kMaxSlices = 8;
+// workgroups (slice_count).
 __device__ __forceinline__ int ragged_m_slices(const TileQueue& q, int nk, bool bf16) {
-  const int by_cu = q.per_xcd > 0 ? q.nbx / q.per_xcd : 1, by_k = nk / kSliceSteps;
-  const float launch = bf16 ? 5.f : 6.5f, part = float(q.n_valid) * (bf16 ? 1.f / 14 : 1.f / 11);
-  int best = 1;
-  float cost = float(nk);
-  for (int s = 2; s <= kMaxSlices && s <= by_cu && s <= by_k; ++s) {
-    const float c = float(nk) / float(s) + launch + part * float(s);
-    if (c < cost) {
-      cost = c;
-      best = s;
-    }
-  }
-  return __builtin_amdgcn_readfirstlane(best);
+  const int by_cu = q.per_xcd > 0 ? q.nbx / q.per_xcd : 1;
+  return __builtin_amdgcn_readfirstlane(slice_count(q.n_valid, by_cu, nk, bf16));
 }
 // A slice's fp32 partial of a tile in the workspace: 256 KiB, wave by wave, 32
 // rows of 64 lanes x 16 bytes (4 consecutive columns i of the row j of the lane).
