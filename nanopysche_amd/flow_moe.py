@@ -950,11 +950,13 @@ class ExpertWeights:
     def views_ok(kind: int, E: int, H: int, D: int, ws, rows: int = 256) -> bool:
         """BF16 recipe on contiguous bf16 parameters, at most 64 experts, H a
         multiple of ``rows``: the row operands are the parameters themselves.
+        On 16-byte boundaries (the GEMM's loads): a parameter that lies elsewhere,
+        as in a flat buffer of many, is copied.
         (The GEMM takes a split at any multiple of 128, as the expert block
         asks for: without it every forward that re-reads its weights, a captured
         one above all, copied them -- 44 us for 8 experts of 2048 x 1408.)"""
         return (ExpertWeights.KMAJOR and kind == _lib.QUANT_BF16 and E <= 64 and H % rows == 0
-                and all(w.dtype == torch.bfloat16 and w.is_contiguous() for w in ws))
+                and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in ws))
 
     def _build_bf16_views(self, w1, w2, w3, E, H, D, dgrad):
         """w13: w1 and w3 read as stored (a split operand), w2: the parameter
