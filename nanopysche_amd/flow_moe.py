@@ -537,12 +537,15 @@ _FEW_CACHED_BYTES = 48 << 20
 
 def _few(plan: RoutingPlan, tokens, w, out) -> bool:
     """Whether a BF16 launch takes fm_grouped_gemm_few: few tokens, in a form that both
-    entries take (what fm_grouped_gemm_ragged_m refuses goes there to be refused)."""
+    entries take (what fm_grouped_gemm_ragged_m refuses goes there to be refused), and an
+    activation of the block, whose padding rows are zeros: that entry writes zeros for
+    a group's padding rows, the other their product."""
+    if type(tokens) is not _Act:
+        return False
     most = _FEW_TOKENS if w.N * w.K * 2 <= _FEW_CACHED_BYTES else _FEW_TOKENS // 2
     if plan.num_tokens > most or plan.num_tokens * plan.top_k > _FEW_PER_EXPERT * plan.num_experts:
         return False
-    t = tokens.buf if type(tokens) is _Act else tokens
-    ld = tokens.ld if type(tokens) is _Act else tokens.stride(0)
+    ld = tokens.ld
     if w.N % 128 or w.K % 128 or w.ld % 16 or w.gs % 8 or w.gs < w.K or ld % 16 or ld < w.K or plan.rows_max == 0:
         return False
     if (w.kmajor or w.data2 is not None) and plan.num_experts > 64:
@@ -552,7 +555,7 @@ def _few(plan: RoutingPlan, tokens, w, out) -> bool:
     if w.data2 is not None and (w.split % (64 if w.kmajor else 128) or not 0 < w.split < (w.K if w.kmajor else w.N)):
         return False
     return (out.stride(0) % 8 == 0 and out.stride(0) >= w.N and not w.paired
-            and not (t.data_ptr() | w.data.data_ptr() | out.data_ptr()
+            and not (tokens.buf.data_ptr() | w.data.data_ptr() | out.data_ptr()
                      | (0 if w.data2 is None else w.data2.data_ptr())) & 15)
 
 

@@ -7,7 +7,7 @@ import torch
 
 import nanopysche_amd as fm
 from nanopysche_amd import _lib
-from nanopysche_amd.flow_moe import ExpertWeightOperand, _dt, _token_operand
+from nanopysche_amd.flow_moe import ExpertWeightOperand, _Act, _dt, _gemm_m, _token_operand
 from tests.helpers import randn_bf16
 
 pytestmark = pytest.mark.gpu
@@ -86,18 +86,38 @@ def test_forms_outside_the_rule_keep_their_kernel(dev, monkeypatch):
     E, N, K = 2, 128, 128
     idx = torch.tensor([[0], [1], [1]], device=dev)
     plan = fm.route_tokens(idx, E)
-    tokens = randn_bf16((plan.rows_max, K), seed=1).to(dev)
+    tokens = fm.fused_permute_pad(randn_bf16((3, K), seed=1).to(dev), plan, E, granularity=None).rows
+    act = _Act(tokens, K, None, 0, False)   # as the block passes them
     W = randn_bf16((E, N, K), seed=2).to(dev)
     w = ExpertWeightOperand(W, None, K, N * K, N=N, K=K)
-    ref = fm.fp8_grouped_gemm(tokens, w, plan)
+    ref = torch.empty(plan.rows_max, N, dtype=torch.bfloat16, device=dev)
     called, real = [], _lib.call
     monkeypatch.setattr(_lib, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    _gemm_m(_lib.QUANT_BF16, act, w, plan, ref)
+    assert called == ["fm_grouped_gemm_few"]
     wide = torch.zeros(plan.rows_max, N + 4, dtype=torch.bfloat16, device=dev)[:, :N]     # pitch 4 mod 8
-    got = fm.fp8_grouped_gemm(tokens, w, plan, out=wide)
-    assert called == ["fm_grouped_gemm_ragged_m"]
+    _gemm_m(_lib.QUANT_BF16, act, w, plan, wide)
+    assert called[1:] == ["fm_grouped_gemm_ragged_m"]
     for e, c in enumerate((1, 2)):
         r = int(plan.offsets[e])
-        assert (got[r:r + c].double() - ref[r:r + c].double()).norm() <= 4e-3 * ref[r:r + c].double().norm()
+        assert (wide[r:r + c].double() - ref[r:r + c].double()).norm() <= 4e-3 * ref[r:r + c].double().norm()
     narrow = ExpertWeightOperand(W[:, :64].contiguous(), None, K, 64 * K, N=64, K=K)
     with pytest.raises(RuntimeError, match="multiple of 128"):
-        fm.fp8_grouped_gemm(tokens, narrow, plan)
+        _gemm_m(_lib.QUANT_BF16, act, narrow, plan, ref)
+
+
+@pytest.mark.parametrize("counts", [(3, 0, 1), (32, 17, 128)])
+def test_public_gemm_multiplies_padding_rows(dev, counts):
+    """fp8_grouped_gemm of a caller's buffer: every row of a group is multiplied, whatever
+    its padding rows hold and however few the tokens."""
+    E, N, K = len(counts), 256, 256
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int64) for e, c in enumerate(counts)])[:, None].to(dev)
+    plan = fm.route_tokens(idx, E)
+    tokens = randn_bf16((plan.rows_max, K), seed=1).to(dev)
+    W = randn_bf16((E, N, K), seed=2, std=0.1).to(dev)
+    out = fm.fp8_grouped_gemm(tokens, ExpertWeightOperand(W, None, K, N * K, N=N, K=K), plan, out_dtype=torch.float32)
+    offs = plan.offsets.tolist()
+    for e in range(E):
+        x, we = tokens[offs[e]:offs[e + 1]].double(), W[e].double()
+        bound = K * 2.0 ** -24 * (x.abs() @ we.abs().t()) + 1e-30
+        assert torch.all((out[offs[e]:offs[e + 1]].double() - x @ we.t()).abs() <= bound)
