@@ -820,6 +820,7 @@ class ExpertWeights:
         self.has_dgrad = False
         self._defer = None
         self.w13 = self.w2t = self.w2 = self.w13t = None
+        self.in_place = ()   # parameters that the operands are (the BF16 views)
 
     def refresh(self, w1, w2, w3, E: int, need_dgrad: bool = True, defer: Optional[list] = None) -> "ExpertWeights":
         """Rebuild the operands if a parameter changed.  With ``defer`` (a list)
@@ -839,6 +840,7 @@ class ExpertWeights:
         if capturing or key != self.key or (need_dgrad and not self.has_dgrad):
             self.key = None
             self.w13 = self.w2t = self.w2 = self.w13t = None
+            self.in_place = ()
             self.has_dgrad = need_dgrad
             self._defer = defer
             try:
@@ -984,6 +986,7 @@ class ExpertWeights:
         if jobs:
             arr = (_lib.FmWeightJob * len(jobs))(*jobs)
             self._launch(arr, len(jobs), w1, (w1, w2, w3))
+        self.in_place = (w1, w2, w3)
         self.w13 = ExpertWeightOperand(w1, None, D, H * D, N=2 * H, K=D, data2=w3, split=H)
         self.w2 = ExpertWeightOperand(w2, None, D, H * D, N=H, K=D)
         if nn:
@@ -1271,6 +1274,9 @@ class FP8FlowMoECompute:
         # the dgrad weight operands of this forward's weights (a later forward
         # may rebuild the cache before this backward runs)
         ctx.dgrad_ops = {k: (ew.w2, ew.w13t) for k, ew in ews.items()} if self._record else None
+        # operands that are the parameters themselves hold this forward's weights
+        # only as long as these do
+        ctx.in_place = tuple((w, w._version) for ew in ews.values() for w in ew.in_place) if self._record else ()
         ctx.saved_hcols = h_cols
         ctx.wdtypes = (w1.dtype, w2.dtype, w3.dtype)
         # Y only feeds the router-weight gradient (the dense path's outputs are
@@ -1290,6 +1296,9 @@ class FP8FlowMoECompute:
         {"addend": bf16 [T, D]}, or with ``can_fold`` {"dlogits": [T, E],
         "gate_w": [E, D]} (E <= 8) for the unpermute to form it itself."""
         wts, GU, Y = ctx.saved_tensors
+        if any(w._version != version for w, version in ctx.in_place):
+            raise RuntimeError("expert weights that the backward reads in place (BF16) were changed by an in-place "
+                               "operation after the forward")
         plan = ctx.plan
         fp8_kind, use_bf16 = ctx.kinds
         E, H, D = self.num_experts, self.hidden_size, self.d_model
