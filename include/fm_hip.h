@@ -245,7 +245,8 @@ int fm_router_logits(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64_
  * of 512 with the gate [8, D] in 64 KiB (D <= 2048 for an fp32 gate, <= 4096
  * for a bf16 one) the gate, gating, loss partials and counts run as one pass
  * over x plus one small kernel (fm_router_forward_fused says which); other
- * gates with bf16 x take three launches, fp32 x the steps separately.  T > 0; the workspace holds
+ * gates with bf16 x take three launches; fp32 x, and gate rows or a workspace off
+ * 16-byte boundaries, the steps separately.  T > 0; the workspace holds
  * fm_router_forward_workspace_bytes(T, E) bytes. */
 int64_t fm_router_forward_workspace_bytes(int64_t T, int E);
 int fm_router_forward_fused(int E, int64_t D, int w_dtype);

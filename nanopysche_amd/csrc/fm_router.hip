@@ -4,7 +4,8 @@
 //                        and logsumexp^2 partials and per-workgroup expert histograms in
 //                        one pass over x, then counts + load-balancing (+ z) loss; in three
 //                        for other gates with bf16 x (the gate's chunk sums, gating and
-//                        partials, counts + loss); fp32 x runs the steps as separate kernels
+//                        partials, counts + loss); fp32 x, or gate rows off 16-byte
+//                        boundaries, run the steps as separate kernels
 //   fm_router_logits     logits[t][e] = sum_d x[t][d] * w[e][d] + bias[e] + score_bias[e], fp32
 //                        (the reference's gate(x.float()) + score_bias, :151-154)
 //   fm_expert_counts     counts[e] = number of the T*K slots routed to e (the f_i of the
@@ -22,7 +23,8 @@
 // its size and the products are summed in fp32, as the reference computes
 // it -- on the matrix cores for bf16 x (bf16 products are exact in fp32, an fp32
 // gate is three exact bf16 pieces, fm_router_mfma.h; the order of the sums
-// differs) except for a small fp32 gate, otherwise as FMAs on the VALU.
+// differs) except for a small fp32 gate and gate rows off 16-byte boundaries, otherwise
+// as FMAs on the VALU.
 // Gate weights are read as stored (fp32 or bf16).
 #include <type_traits>
 
@@ -1036,6 +1038,11 @@ inline bool router_small_ok(int E, int64_t D, int w_bf16) {
   return E <= 8 && D % kRouterCols == 0 && 8 * D * (w_bf16 ? 2 : 4) <= kGateLdsBytes;
 }
 
+// gate_logits_kernel reads the gate's rows 16 bytes at a time; a bf16 gate's may
+// lie on 8 (a pitch of 4 mod 8 elements, a view into a buffer), where the FMA
+// kernel's loads are of that size.
+inline bool gate_rows16(const RouterArgs& a) { return aligned16(a.w) && a.ld_w % (a.w_bf16 ? 8 : 4) == 0; }
+
 // bf16 x: the gate on the matrix cores, as chunk sums (SPLIT: out = part) or logits.
 template <bool SPLIT>
 int gate_logits_launch(const RouterArgs& r, float* out, int64_t ld_o, hipStream_t s, const char* what) {
@@ -1080,12 +1087,16 @@ int router_logits_launch(const RouterArgs& a, int x_dtype, const RouterFuse* f, 
       else { if (xb) FM_SMALL(uint16_t, float, false); else FM_SMALL(float, float, false); }
     }
 #undef FM_SMALL
-  } else if (xb) {
+  } else if (xb && gate_rows16(a)) {
     return gate_logits_launch<false>(a, a.logits, a.ld_l, s, what);
   } else if (a.E <= 8) {
-    hipLaunchKernelGGL((router_logits_kernel<float, 8>), dim3(rb, 1), dim3(256), 0, s, a);
+    const dim3 grid(rb, 1);
+    if (xb) hipLaunchKernelGGL((router_logits_kernel<uint16_t, 8>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((router_logits_kernel<float, 8>), grid, dim3(256), 0, s, a);
   } else {
-    hipLaunchKernelGGL((router_logits_kernel<float, 16>), dim3(rb, unsigned((a.E + 15) / 16)), dim3(256), 0, s, a);
+    const dim3 grid(rb, unsigned((a.E + 15) / 16));
+    if (xb) hipLaunchKernelGGL((router_logits_kernel<uint16_t, 16>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((router_logits_kernel<float, 16>), grid, dim3(256), 0, s, a);
   }
   return check_launch(what);
 }
@@ -1228,9 +1239,9 @@ int fm_router_forward(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64
                        total_tokens, T, part, zm != 0.f ? zpart : nullptr, zm, loss);
     return check_launch("fm_router_forward");
   }
-  // other gates with bf16 x: the gate's chunk sums, the gating (which adds them),
-  // and counts + loss
-  if (x_dtype == FM_DTYPE_BF16) {
+  // other gates with bf16 x: the gate's chunk sums (stored 16 bytes at a time), the
+  // gating (which adds them), and counts + loss
+  if (x_dtype == FM_DTYPE_BF16 && gate_rows16(a) && aligned16(workspace)) {
     const GateShape g = gate_shape(T, D, E, w_dtype != FM_DTYPE_BF16);
     const int64_t gb = gate_blocks(T);
     float* prob = base + g.S * T * g.ld_p;
@@ -1252,7 +1263,8 @@ int fm_router_forward(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64
                        total_tokens, T, prob, zm != 0.f ? zp : nullptr, zm, loss);
     return check_launch("fm_router_forward");
   }
-  // fp32 x: logits, then gating, counts and loss as separate kernels
+  // fp32 x, or a gate or workspace off 16 bytes: logits, then gating, counts and
+  // loss as separate kernels
   float* part = base;
   float* zpart = base + kRouterForwardWaves * E;
   if (int rc = router_logits_launch(a, x_dtype, nullptr, 0, s, "fm_router_forward")) return rc;

@@ -62,6 +62,29 @@ def test_products_at_tile_edges(dev, T, D, E, gate):
     assert torch.equal(only, dx)
 
 
+@pytest.mark.parametrize("pitch,start", [(4, 0), (0, 4), (12, 4)])
+@pytest.mark.parametrize("T,D,E", [(33, 264, 33), (37, 200, 5), (100, 4104, 3), (64, 512, 64)])
+def test_gate_rows_off_16_bytes(dev, T, D, E, pitch, start):
+    """A bf16 gate whose rows lie on 8 bytes keeps the FMA kernel: the bits of the fp32-x
+    path (the same values, read wider), in the logits and in the whole forward."""
+    g, x, w, b, sb = _inputs(dev, T, D, E, torch.bfloat16)
+    flat = torch.zeros(E * (D + pitch) + 8, dtype=torch.bfloat16, device=dev)
+    view = flat[start:start + E * (D + pitch)].view(E, D + pitch)[:, :D]
+    view.copy_(w)
+    assert flat.data_ptr() % 16 == 0 and (view.data_ptr() % 16 or 2 * view.stride(0) % 16)
+    ref = fm.router_logits(x.float(), view, b, sb)
+    assert torch.equal(fm.router_logits(x, view, b, sb), ref)
+    K = min(E, 4)
+    got = router_forward(x, view, b, sb, K, "sigmoid", None, None, 1e-3)
+    want = router_forward(x.float(), view, b, sb, K, "sigmoid", None, None, 1e-3)
+    for u, v in zip((*got[:3], got[3].logits, got[3].counts), (*want[:3], want[3].logits, want[3].counts)):
+        assert torch.equal(u, v)
+    dws, daux = torch.randn(T, K, generator=g).to(dev), torch.tensor(0.5, device=dev)
+    for u, v in zip(router_backward(got[3], x, view, dws, daux, bias_dtype=torch.float32),
+                    router_backward(got[3], x, w, dws, daux, bias_dtype=torch.float32)):
+        assert torch.equal(u, v)
+
+
 @pytest.mark.parametrize("T,D,E", [(40, 136, 9), (64, 264, 40), (64, 4104, 3)])
 def test_dx_of_fp32_factors_has_every_product(dev, T, D, E):
     """dlogits a and gate b, all low mantissa bits set, in expert 0; the product's two
