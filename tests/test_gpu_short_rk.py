@@ -27,6 +27,8 @@ def _wide(t, ld, paired):
     ([0, 100, 128, 129, 384, 700], 384, 1152, False),     # 0 .. 6 K steps of 128; a 9th tile column, 3 tile rows
     ([300], 256, 128, False),                             # one expert, fewer tiles than a chunk
     ([1, 0, 513, 0, 40, 256, 200, 90], 256, 1024, True),
+    ([0, 1, 128, 200] * 16, 256, 128, False),             # as many experts as lanes, the first without tokens
+    ([130, 0, 40, 257] * 16, 256, 256, True),
 ])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
 def test_few_token_weight_gradient_bits(dev, kind, paired, counts, M, N, masked, out):
