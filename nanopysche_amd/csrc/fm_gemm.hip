@@ -2839,22 +2839,32 @@ int prepare_gemm(int kind, GemmParams& p) {
 
 // Ragged-K launches of few tokens per expert take the 128 x 128 kernel: at most
 // 512 padded tokens an expert on average, or 1152 where an expert's gradient has
-// 2^25 elements or more (`p` as prepared; the operands' pitch bounds the tokens).
-// Measured over a training step, 256 x 256 kernels against this one, at 128 /
-// 256 / 384 / 512 / 1024 tokens per expert: 8 experts of 4096 x 14336 (pow2) 2553
-// / 2826 / 3155 / 3886 / 5711 us against 2409 / 2659 / 3030 / 3727 / 5536 (bf16
-// 3327 / 3930 / 4492 / 6269 / 10493 against 3109 / 3756 / 4288 / 6192 / 10234), 8
-// experts of 2048 x 1408 (pow2) 286 / 301 / 325 / 330 / 469 against 271 / 286 /
-// 316 / 345 / 485, 64 such experts (bf16) 1399 / 1934 / 2288 / 2682 / 4587 against
-// 1320 / 1852 / 2285 / 2632 / 4589.  The larger tiles reuse operands better, which
-// counts from about 512 tokens on, later where the operands of an expert's tiles
-// in flight leave an XCD's L2 either way.
-constexpr int64_t kShortRows = 512, kShortRowsLarge = 1152, kShortLarge = int64_t(1) << 25;
+// 2^25 elements or more (896 for pow2 without a mask, which the paired ring walks
+// faster; `p` as prepared; the operands' pitch bounds the tokens).  Measured over a training
+// step of 8 experts, dW1 | dW3 and dW2 on the 256 x 256 kernels against this one, us:
+//   tokens an expert         256          512          640          768          1024
+//   1408 x 2048 pow2     301 / 286    330 / 345                               469 / 485
+//   2048 x 7168 pow2     788 / 738   1019 / 1024  1106 / 1115  1170 / 1190  1516 / 1542
+//               bf16    1339 / 1290  1856 / 1848  2020 / 2009  2281 / 2267  2986 / 2974
+//   4096 x 4096 pow2     789 / 773   1108 / 1071  1272 / 1215  1341 / 1306  1693 / 1696
+//               bf16    1276 / 1224  1975 / 1935  2265 / 2153  2482 / 2388  3183 / 3153
+//   8192 x 4096 pow2    1268 / 1241  1996 / 1952  2223 / 2154  2376 / 2375  3021 / 3088
+//               bf16    2247 / 2206  3737 / 3597  4116 / 3986  4548 / 4471  6009 / 5989
+//   12288 x 4096 pow2   1868 / 1842  2848 / 2792  3155 / 3100  3429 / 3428  4387 / 4442
+//               bf16    3530 / 3442  5751 / 5567  6385 / 6112  6973 / 6860  9074 / 9020
+//   14336 x 4096 pow2   2182 / 2066  3322 / 3170  3653 / 3523  4073 / 3982  5130 / 5113
+//               bf16    3871 / 3710  6666 / 6437  7373 / 7029  8084 / 7835 10624 / 10408
+// and a masked launch alone (28672 x 4096, half of 8 experts), at 1024 tokens 1.17 (bf16) and
+// 1.09 (pow2) times as fast.  The larger tiles reuse operands better, which counts
+// from about 512 tokens on, later where the operands of an expert's tiles in flight
+// leave an XCD's L2 either way.
+constexpr int64_t kShortRows = 512, kShortRowsLarge = 1152, kShortRowsRing = 896, kShortLarge = int64_t(1) << 25;
 inline bool gemm_rk_short(int kind, const GemmParams& p) {
   const int64_t row = p.out_f32 ? 4 : 8;   // elements of a 16-byte store
   const bool aligned = p.ldC % row == 0 && p.c_gs % row == 0 && (size_t(p.C) & 15) == 0 &&
                        (p.split == INT64_MAX || (p.c2_gs % row == 0 && (size_t(p.C2) & 15) == 0));
-  const int64_t rows = p.n_i * p.n_j >= kShortLarge ? kShortRowsLarge : kShortRows;
+  const int64_t large = kind == GK_FP8_POW2 && p.mask == nullptr ? kShortRowsRing : kShortRowsLarge;
+  const int64_t rows = p.n_i * p.n_j >= kShortLarge ? large : kShortRows;
   return (kind == GK_BF16 || kind == GK_FP8_POW2) && p.splits == 1 && p.E <= 64 && aligned &&
          p.P.ld <= rows * p.E && p.n_tiles < (int64_t(1) << 24);
 }
