@@ -602,11 +602,16 @@ def _m_split(kind, plan: RoutingPlan, w: ExpertWeightOperand, out, mask) -> bool
     """A ragged-M launch (BF16, or paired FP8) that is expected to leave at
     least half of the CUs without a tile and whose K is long enough for the
     partials' round trip: the device then slices K by the tiles that there are
-    (ragged_m_slices, whose costs these are).  Under an expert mask the tiles
-    are not known: any BF16 launch (its experts are those with few tokens) of 64
-    steps, or 88 with more than 512 tokens an expert (steps of half of 8 experts of
-    2048 x 5632 in BF16, 2048 / 8192 tokens, 1566 / 2960 us against 1291 / 2850; 16
-    of 1024 x 4096 with 1024 each 1890 against 1902 with 64 for all).  Measured unsliced against sliced, [K][N] weights, tokens over all
+    (slice_count, whose costs these are).  Under an expert mask the tiles are not
+    known: any BF16 launch (its experts are those with few tokens) of 64 steps, or
+    88 with more than 512 tokens an expert, which leave more tiles.  Over 1200 masked
+    launches (4 to 32 experts, N 1024 to 4096, K of 16 to 224 steps, Zipf 0.6 and
+    1.1, the experts below the mean in BF16) sliced ones are, with up to 512 tokens
+    an expert, on average 1.34 times as fast at 48 steps, but 0.76 times at worst (128
+    tiles, 2 slices on all CUs), 1.47 and 0.90 at 64, 1.5 to 2 and 0.95 from 72 on; with
+    more tokens 1.13 and 0.91 at 64, 1.24 and 0.89 at 80, 1.18 and 0.94 at 88, 1.41 and
+    0.95 from 96 on.
+    Measured unsliced against sliced, [K][N] weights, tokens over all
     experts 512 / 1024 / 2048: BF16, 8 experts of K 5632, N 2048, 128 / 139 /
     140 us against 59 / 70 / 99; of K 2048 38 / 40 / 42 against 33 / 40 / 49 (not
     sliced); 8 of K 14336, N 4096, at 512 / 1024 351 / 393 against 228 / 265; pow2
