@@ -521,7 +521,8 @@ typedef struct FmGemmOperand {
  * dgrad): out[r][n] = sum_k tokens[r][k] * weights_e[n][k] for the rows r of
  * expert e, offsets[e] <= r < offsets[e+1] (offsets and tile_expert as written
  * by fm_route_sort: [E+1] padded group starts and the expert of each 128-row
- * tile, -1 past the last group).  Experts with expert_mask[e] != mask_want
+ * tile, -1 past the last group; tile_expert must be given, but the kernels find
+ * their tiles from the offsets).  Experts with expert_mask[e] != mask_want
  * when expert_mask != NULL are skipped -- the fp8_gemm_threshold switch of
  * model/moe.py:1215-1216.  N, K multiples of 128. */
 int fm_grouped_gemm_ragged_m(int kind, const FmGemmOperand* tokens, const FmGemmOperand* weights,

@@ -100,6 +100,10 @@ FM_HD uint8_t quant_e4m3(float x, float scale) { return f32_to_e4m3(clamp448(x /
 typedef uint32_t fm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t fm_u32x4 __attribute__((ext_vector_type(4)));
 typedef float fm_f32x4 __attribute__((ext_vector_type(4)));
+// operands and accumulators of the bf16 MFMAs and of the transposing LDS reads
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef short v4s16 __attribute__((ext_vector_type(4)));
 #define FM_GLOBAL(T, p) ((__attribute__((address_space(1))) T*)(p))
 __device__ __forceinline__ void st_global(void* p, uint4 v) { *FM_GLOBAL(fm_u32x4, p) = fm_u32x4{v.x, v.y, v.z, v.w}; }
 __device__ __forceinline__ void st_global(void* p, uint2 v) { *FM_GLOBAL(fm_u32x2, p) = fm_u32x2{v.x, v.y}; }

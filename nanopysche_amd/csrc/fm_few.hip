@@ -20,10 +20,6 @@
 
 namespace fm {
 
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef short v4s16 __attribute__((ext_vector_type(4)));
-
 constexpr int kFewRows = 64;     // weight rows of a workgroup
 constexpr int kFewTokens = 32;   // tokens of a pass
 

@@ -53,7 +53,6 @@ namespace fm {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 enum GemmKind : int { GK_BF16 = 0, GK_FP8_F32 = 1, GK_FP8_POW2 = 2, GK_FP8_MX = 3 };
 enum GemmMode : int { GM_RAGGED_M = 0, GM_RAGGED_K = 1 };
@@ -76,7 +75,6 @@ struct GemmParams {
   int64_t n_i;        // extent of i (rows of Q per group)
   int64_t n_j;        // ragged-K: extent of j (rows of P)
   int64_t K;          // ragged-M: contraction length
-  const int32_t* tile_expert;  // ragged-M: expert of each 128-row tile
   int64_t m_tiles;             // ragged-M: 128-row tiles in the padded buffer
   int64_t j_tiles;             // ragged-M, 256 x 256 kernel: bound on 256-row token tiles
   const int32_t* offsets;      // [E+1] padded group starts (rows)
@@ -110,30 +108,20 @@ __device__ __forceinline__ int lds_off(int row, int chunk) {
   return row * 128 + ((chunk ^ lds_swz(row)) << 4);
 }
 
-// LDS-DMA: the 64 lanes' `size`-byte loads land at consecutive LDS addresses
-// starting at `lds` (wave-uniform); `g` is each lane's own global source.
-// Issued from inline assembly so the compiler's wait insertion does not treat
-// them as pending LDS writes (it would wait for every prefetch in flight before
-// each LDS read); the kernels order them with explicit vmcnt waits instead.
+// LDS-DMA: the 64 lanes' loads land at consecutive LDS addresses starting at
+// `lds` (wave-uniform).  Issued from inline assembly so the compiler's wait
+// insertion does not treat them as pending LDS writes (it would wait for every
+// prefetch in flight before each LDS read); the kernels order them with explicit
+// vmcnt waits instead.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return uint32_t(size_t((__attribute__((address_space(3))) const void*)(p)));
 }
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is written here and nowhere else
-__device__ __forceinline__ void dma16(const void* g, const void* lds) {
-  const uint32_t m = __builtin_amdgcn_readfirstlane(lds_addr(lds));
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(m) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4a(const void* g, uint32_t lds) {
-  const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(m) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void* g, const void* lds) { dma4a(g, lds_addr(lds)); }
-// Buffer-resource form, the 256 x 256 kernel's path: a raw-buffer descriptor
-// of a wave-uniform base (the wave's first row of the tile), a 32-bit
-// per-lane offset and a 32-bit uniform offset (group + K position), so no
-// 64-bit address arithmetic is spent per load.  Measured on gfx950 it moves
-// the tile's 64 KiB per K step at the same rate as the flat form.
+// A raw-buffer descriptor of a wave-uniform base (the wave's first row of the
+// tile), a 32-bit per-lane offset and a 32-bit uniform offset (group + K
+// position), so no 64-bit address arithmetic is spent per load.  Measured on
+// gfx950 it moves the tile's 64 KiB per K step at the same rate as the flat form.
 // byte address = base + voff + soff.
 __device__ __forceinline__ void bdma16(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
@@ -184,7 +172,7 @@ __device__ __forceinline__ void block_barrier() {
 }
 
 // ============================================================================
-// 256 x 256 kernel: BF16, FP8_POW2, FP8_MX
+// 256 x 256 kernel
 // ============================================================================
 constexpr int kT = 256;
 
@@ -313,7 +301,6 @@ __device__ __forceinline__ v8i read_frag8_nn(const uint8_t* st, int ibase, int h
   return f;
 }
 
-typedef short v4s16 __attribute__((ext_vector_type(4)));
 // ds_read_b64_tr_b16 (gfx950): in each 16-lane group, lane 4r + p gives the
 // address of elements [4p, 4p + 4) of row r (r = 0..3), and lane m of the
 // group receives element m of every row (4 elements, row order).  Established
@@ -3053,7 +3040,6 @@ int ragged_m_params(int kind, int nn, int paired, const FmGemmOperand* tokens, c
   p.Q = make_operand(*weights);
   p.n_i = N;
   p.K = K;
-  p.tile_expert = tile_expert;
   p.m_tiles = m_tiles;
   // sum over experts of ceil(tiles_e / 2) <= (m_tiles + E) / 2
   p.j_tiles = (m_tiles + E + 1) / 2;

@@ -24,10 +24,6 @@
 
 namespace fm {
 
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef short v4s16 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ v4f mfma16(const uint4& a, const uint4& b, v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }

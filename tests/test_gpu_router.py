@@ -207,8 +207,8 @@ def _separate(x, w, b, sb, K, gating, replay, normalize, z_mult):
     (1000, 512, 4, 2, "sigmoid", False, "l2", 1e-3),
     (333, 1536, 8, 8, "softmax", True, None, 1e-2),
     (77, 512, 1, 1, "softmax", False, None, 0.0),
-    (500, 256, 8, 2, "softmax", False, None, 0.0),       # D not a multiple of 512: separate kernels
-    (300, 512, 24, 4, "sigmoid", True, "l2", 1e-3),      # E > 8: separate kernels
+    (500, 256, 8, 2, "softmax", False, None, 0.0),       # D not a multiple of 512: three launches
+    (300, 512, 24, 4, "sigmoid", True, "l2", 1e-3),      # E > 8: three launches
 ])
 @pytest.mark.parametrize("w_dtype", [torch.float32, torch.bfloat16])
 def test_fused_router_forward_matches_separate_kernels(dev, T, D, E, K, gating, replay, normalize, z_mult, w_dtype):
