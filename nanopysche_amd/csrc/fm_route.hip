@@ -44,6 +44,7 @@ __device__ __forceinline__ void topk_logits(const TopkArgs& a, int64_t t, int e,
     int c[NJ];   // experts past E read the last one
 #pragma unroll
     for (int j = 0; j < NJ; ++j) c[j] = e + 64 * j < a.E ? e + 64 * j : a.E - 1;
+    double d[NJ];
     for (int64_t s = 0; s < a.S; s += 8) {
       float u[8][NJ];
 #pragma unroll
@@ -54,10 +55,11 @@ __device__ __forceinline__ void topk_logits(const TopkArgs& a, int64_t t, int e,
       for (int i = 0; i < 8; ++i)
         if (s + i < a.S)
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) v[j] = s + i == 0 ? u[0][j] : v[j] + u[i][j];
+          for (int j = 0; j < NJ; ++j) d[j] = s + i == 0 ? double(u[0][j]) : d[j] + double(u[i][j]);
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
+      v[j] = float(d[j]);
       if (a.bias)
         v[j] += a.bias_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(a.bias)[c[j]]) : static_cast<const float*>(a.bias)[c[j]];
       if (a.score_bias) v[j] += a.score_bias[c[j]];

@@ -1046,26 +1046,42 @@ inline bool gate_rows16(const RouterArgs& a) { return aligned16(a.w) && a.ld_w %
 // bf16 x: the gate on the matrix cores, as chunk sums (SPLIT: out = part) or logits.
 template <bool SPLIT>
 int gate_logits_launch(const RouterArgs& r, float* out, int64_t ld_o, hipStream_t s, const char* what) {
-  const GateShape g = gate_shape(r.T, r.D, r.E, !r.w_bf16);
+  GateShape g = gate_shape(r.T, r.D, r.E, !r.w_bf16);
+  if (!SPLIT && g.tf > 2) {   // registers for the sum over chunks; an output's bits depend on the chunks alone
+    g.tf = 2;
+    g.tt = (r.T + 31) / 32;
+  }
   const GateLogitsArgs a{static_cast<const uint16_t*>(r.x), r.ld_x, r.T, r.D, r.w, r.ld_w, r.bias, r.score_bias, r.E,
-                         g.S, g.chunk, g.eg, int(g.tt), out, ld_o};
+                         g.S, g.chunk, g.eg, int(g.tt), gate_group_columns(r.D, !r.w_bf16) - 64, out, ld_o};
   const int64_t waves = g.tt * g.eg * (SPLIT ? g.S : 1);
   const dim3 grid{unsigned((waves + 3) / 4)}, block{256};
-#define FM_GATE(TF, NF, W) hipLaunchKernelGGL((gate_logits_kernel<TF, NF, W, SPLIT>), grid, block, 0, s, a)
-#define FM_GATE_NF(TF, W)              \
-  switch (g.nf) {                      \
-    case 1: FM_GATE(TF, 1, W); break;  \
-    case 2: FM_GATE(TF, 2, W); break;  \
-    case 3: FM_GATE(TF, 3, W); break;  \
-    default: FM_GATE(TF, 4, W); break; \
-  }
+  auto launch = [&](auto tf, auto nf, auto w32) {
+    hipLaunchKernelGGL((gate_logits_kernel<decltype(tf)::value, decltype(nf)::value, decltype(w32)::value, SPLIT>),
+                       grid, block, 0, s, a);
+  };
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  constexpr std::integral_constant<int, 3> three;
+  constexpr std::integral_constant<int, 4> four;
+  auto tokens = [&](auto nf, auto w32) {
+    if constexpr (SPLIT && !decltype(w32)::value && decltype(nf)::value < 4) {
+      if (g.tf == 4) return launch(four, nf, w32);
+    }
+    if (g.tf == 1) launch(one, nf, w32);
+    else launch(two, nf, w32);
+  };
   if (r.w_bf16) {
-    if (g.tf == 1) FM_GATE_NF(1, false) else if (g.tf == 2) FM_GATE_NF(2, false) else FM_GATE_NF(4, false)
+    switch (g.nf) {
+      case 1: tokens(one, std::false_type{}); break;
+      case 2: tokens(two, std::false_type{}); break;
+      case 3: tokens(three, std::false_type{}); break;
+      default: tokens(four, std::false_type{}); break;
+    }
+  } else if (g.nf == 1) {
+    tokens(one, std::true_type{});
   } else {
-    if (g.tf == 1) FM_GATE_NF(1, true) else FM_GATE_NF(2, true)
+    tokens(two, std::true_type{});
   }
-#undef FM_GATE_NF
-#undef FM_GATE
   return check_launch(what);
 }
 

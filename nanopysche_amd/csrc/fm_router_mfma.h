@@ -4,8 +4,9 @@
 //   dw     = dlogits^T x  (gate_dw_kernel)
 // with the fp32 operand of each (dlogits, an fp32 gate) as three bf16 pieces
 // whose sum is the value exactly (8 + 8 + 8 mantissa bits), so every product
-// is exact in the fp32 accumulator and the results are fp32 sums of exact
-// products as on the VALU, in another order.
+// is exact in the fp32 accumulator and the results are sums of exact products
+// as on the VALU, in another order (fp32 within a chain of MFMAs, each section below
+// says how the chains' sums are added).
 //
 // Non-finite values: the two low pieces of an infinity or a NaN are 0, and the
 // low pieces' sum is dropped where it is not finite (an infinite factor on
@@ -60,9 +61,16 @@ __device__ __forceinline__ float finite_or_0(float v) { return fabsf(v) <= 3.402
 // touch four lines per four lanes: 65 us for [4096, 7168] x 256 experts,
 // bound by the L1's tag rate.)  Row i of expert fragment f stands for expert
 // e0 + 4 NF (i / 4) + 4 f + i % 4, so a lane ends with 4 NF consecutive experts
-// of one token.  The chunks' sums are added in chunk order, by the gating kernel
-// (SPLIT: the chunk's sums go to part [S][T][ld_p]) or by this wave over all
+// of one token.  The chunks' sums are added in chunk order in 64 bits, by the gating
+// kernel (SPLIT: the chunk's sums go to part [S][T][ld_p]) or by this wave over all
 // chunks (SPLIT false), with the same bits.
+// The MFMA chains are short (gate_group_columns): a chain's sums join the chunk's
+// with the remainder of that rounding carried into the next chain (compensated
+// summation), where one chain a chunk and fp32 sums of the chunks were less exact
+// than the FMAs' 64 lane sums.  Rms error against float64 in units of the logits',
+// FMAs / one chain a chunk / now: bf16 gate, 16384 tokens, [1024] x 256 6.8e-8 /
+// 1.3e-7 / 5.2e-8, [7168] x 256 9.5e-8 / 3.7e-7 / 6.6e-8, [7168] x 12 9.5e-8 / 1.8e-7 /
+// 7.1e-8; fp32 gate, [7168] x 256 2.0e-7 / 5.3e-7 / 9.0e-8.
 struct GateLogitsArgs {
   const uint16_t* x;     // bf16 [T, ld_x]
   int64_t ld_x, T, D;
@@ -73,12 +81,13 @@ struct GateLogitsArgs {
   int E;
   int64_t S, chunk;      // chunk: a multiple of 64
   int eg, tt;            // expert groups, token tiles
+  int group;             // columns of an MFMA chain, less 64 (bits above 6)
   float* out;            // SPLIT: part [S][T][ld_o]; else logits [T, ld_o]
   int64_t ld_o;
 };
 
 template <int TF, int NF, bool W32, bool SPLIT>
-__global__ __launch_bounds__(256) void gate_logits_kernel(GateLogitsArgs a) {
+__global__ __launch_bounds__(256, SPLIT ? 2 : 1) void gate_logits_kernel(GateLogitsArgs a) {
   constexpr int XR = 16 * TF, WR = 16 * NF * (W32 ? 2 : 1);   // 128-byte rows: tokens; experts (fp32: halves of 32 columns)
   __shared__ __attribute__((aligned(16))) uint8_t lds[4][(XR + WR) * 128];
   const int lane = threadIdx.x & 63, m = lane & 15, q = lane >> 4;
@@ -143,6 +152,8 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(GateLogitsArgs a) {
     return *reinterpret_cast<const uint4*>(mine + (XR + r) * 128 + ((c ^ (r >> (W32 ? 2 : 1))) & 7) * 16);
   };
   v4f tot[NF][TF];
+  typedef double v4d __attribute__((ext_vector_type(4)));
+  v4d all[SPLIT ? 1 : NF][SPLIT ? 1 : TF];   // the chunks' sums (topk_logits adds those of SPLIT, alike)
   for (int64_t s = s0; s < (SPLIT ? s0 + 1 : a.S); ++s) {
     const int64_t k0 = s * a.chunk, k1 = k0 + a.chunk < a.D ? k0 + a.chunk : a.D;
     v4f acc[NF][TF], low[W32 ? NF : 1][W32 ? TF : 1];
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(GateLogitsArgs a) {
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int t = 0; t < TF; ++t) {
-        acc[f][t] = v4f{0.f, 0.f, 0.f, 0.f};
+        acc[f][t] = tot[f][t] = v4f{0.f, 0.f, 0.f, 0.f};
         if constexpr (W32) low[f][t] = v4f{0.f, 0.f, 0.f, 0.f};
       }
     load(k0, k1);
@@ -182,16 +193,28 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(GateLogitsArgs a) {
           }
         }
       }
+      // the group's sums into the chunk's; what that rounding drops starts the next group's
+      if (((k - k0) & a.group) != a.group && k + 64 < k1) continue;
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int t = 0; t < TF; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float v = tot[f][t][i] + acc[f][t][i];
+            acc[f][t][i] = finite_or_0((tot[f][t][i] - v) + acc[f][t][i]);
+            tot[f][t][i] = v;
+          }
     }
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
-      for (int t = 0; t < TF; ++t) {
-        if constexpr (W32)
+      for (int t = 0; t < TF; ++t)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[f][t][i] += finite_or_0(low[f][t][i]);
-        tot[f][t] = s == s0 ? acc[f][t] : tot[f][t] + acc[f][t];
-      }
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (W32) tot[f][t][i] += acc[f][t][i] + finite_or_0(low[f][t][i]);
+          if constexpr (!SPLIT) all[f][t][i] = s == s0 ? double(tot[f][t][i]) : all[f][t][i] + double(tot[f][t][i]);
+        }
   }
 #pragma unroll
   for (int t = 0; t < TF; ++t) {
@@ -209,7 +232,7 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(GateLogitsArgs a) {
         for (int i = 0; i < 4; ++i) {
           const int e = eb + 4 * f + i;
           if (e < a.E) {
-            float v = tot[f][t][i];
+            float v = float(all[f][t][i]);
             if (a.bias) v += W32 ? static_cast<const float*>(a.bias)[e] : bf16_to_f32(static_cast<const uint16_t*>(a.bias)[e]);
             if (a.score_bias) v += a.score_bias[e];
             a.out[tok * a.ld_o + e] = v;
@@ -229,8 +252,8 @@ struct GateShape {
 };
 inline GateShape gate_shape(int64_t T, int64_t D, int E, bool w32) {
   GateShape g;
-  g.nf = E <= 16 ? 1 : E <= 32 ? 2 : E <= 48 ? 3 : 4;
-  g.tf = T <= 16 ? 1 : (T <= 32 || w32) ? 2 : 4;   // an fp32 gate: two sums per output
+  g.nf = E <= 16 ? 1 : E <= 32 || w32 ? 2 : E <= 48 ? 3 : 4;   // an fp32 gate: two sums per output
+  g.tf = T <= 16 ? 1 : (T <= 32 || w32 || g.nf == 4) ? 2 : 4;
   g.eg = (E + 16 * g.nf - 1) / (16 * g.nf);
   g.tt = (T + 16 * g.tf - 1) / (16 * g.tf);
   int64_t s = 2048 / (g.tt * g.eg);
@@ -246,6 +269,14 @@ inline GateShape gate_shape(int64_t T, int64_t D, int E, bool w32) {
   g.ld_p = int64_t(g.eg) * 16 * g.nf;
   return g;
 }
+
+// Columns of an MFMA chain: short enough that the rms error is below the FMA
+// kernel's at every D.  FMAs, chains of 64, 128 and 256 columns, bf16 gate (16384
+// tokens): D 384 5.9e-8, 5.7e-8, (chunk) 6.9e-8; 1024 6.8e-8, 5.7e-8, 7.0e-8; 4096 8.4e-8,
+// 5.8e-8, 7.1e-8, 9.4e-8; fp32 gate: D 512 8.6e-8, 5.7e-8, 6.9e-8, 9.0e-8; 2560 1.3e-7, 5.7e-8, 7e-8, 9e-8.
+// A join is five VALU instructions a sum: forward of [4096, 7168] x 256 with 64 / 128 / 256
+// columns 80 / 75 / 72 us.
+inline int gate_group_columns(int64_t D, bool w32) { return (D < 2048 ? 64 : 128) << int(w32); }
 
 // ------------------------------------------- pieces for the backward ----
 // Tiles of 64 x 64: dlogits [T, E] into its bf16 pieces by token (p, [3][Tp x Ep],

@@ -5,7 +5,7 @@ slices of tokens.
 
 Bounds: every product of pieces is exact in fp32, so a sum over n is off by at
 most (n + 2) 2^-24 sum |terms|, the 2 for the low pieces joining the high ones
-(n 2^-23 for the nine pairs of pieces of two fp32 factors)."""
+(n 2^-23 for the nine pairs of pieces of two fp32 factors), whatever its order."""
 
 import pytest
 import torch
@@ -111,6 +111,25 @@ def test_dx_of_fp32_factors_has_every_product(dev, T, D, E):
               _lib.DTYPE_F32, D, E, _lib.addr(dx), D, None, _lib.DTYPE_F32, 0, None, _lib.DTYPE_F32, _lib.addr(ws),
               ws.numel(), _lib.stream_of(x))
     assert float(dx.diagonal()[:n].abs().max()) <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
+def test_logits_keep_small_terms_beside_a_large_one(dev, gate):
+    """2^25 first, -2^25 last and 30 ones between, one in each step of 64 columns, in one
+    chunk of D: 30.  A chain of MFMAs is at most 256 columns; the large term's ulp of 4 swallows the
+    ones of its own chain (at most 3 of the first, and 4 of the last with two roundings of at
+    most 2), never those carried between chains.  One chain over all columns gives 0."""
+    T, D, E = 16384, 2048, 256
+    x, w = torch.zeros(T, D, dtype=torch.bfloat16, device=dev), torch.zeros(E, D, dtype=gate, device=dev)
+    x[:, 65:D - 64:64] = 1
+    w[:, 65:D - 64:64] = 1
+    x[:, 0], x[:, D - 1] = 2.0 ** 12, -(2.0 ** 12)
+    w[:, 0] = w[:, D - 1] = 2.0 ** 13
+    ref = float(x[0].double() @ w[0].double())
+    assert ref == 30
+    got = router_forward(x, w, None, None, 4, "softmax", None, None, 0.0)[3].logits
+    assert float((got - ref).abs().max()) <= 11
+    assert torch.equal(fm.router_logits(x, w), got)
 
 
 @pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
