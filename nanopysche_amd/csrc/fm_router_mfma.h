@@ -319,9 +319,9 @@ __global__ __launch_bounds__(256) void gate_pieces_kernel(GatePieceArgs a) {
     }
     __syncthreads();
     if (a.db_part && r4 == 0 && e0 + c < a.E) {
-      float s = 0.f;
-      for (int r = 0; r < 64; ++r) s += tile[r][c];
-      a.db_part[int64_t(blockIdx.x) * a.E + e0 + c] = s;
+      double s = 0.;
+      for (int r = 0; r < 64; ++r) s += double(tile[r][c]);
+      a.db_part[int64_t(blockIdx.x) * a.E + e0 + c] = float(s);
     }
     const int row = tid >> 2, col = (tid & 3) * 16;
 #pragma unroll
@@ -607,7 +607,10 @@ __global__ __launch_bounds__(256, 2) void gate_dw_kernel(GateDwArgs a) {
 
 // dw = the slices' partials summed in slice order (four columns a thread, eight
 // slices' loads in flight); an expert's last workgroup its db = the token tiles'
-// column sums (lane-strided tiles, then a fixed shuffle tree).
+// column sums (lane-strided tiles, then a fixed shuffle tree).  Both in 64 bits,
+// as the tiles' column sums: up to 64 partials of a few MFMAs each, and 64 tokens, one
+// after the other in fp32 were less exact than the VALU kernels' sums (rms error of dw,
+// 16384 tokens, [1024] x 12: 1.6e-7 there, 1.9e-7 in fp32, 1.2e-7 now; db 2 to 3 times).
 struct GateDwSumArgs {
   const float* part;
   int64_t S, D;
@@ -627,11 +630,12 @@ __global__ __launch_bounds__(256) void gate_dw_sum_kernel(GateDwSumArgs a) {
     if (a.db == nullptr) return;
     const int lane = threadIdx.x & 63, e = blockIdx.y;
     if (threadIdx.x < 64) {
-      float v = 0.f;
+      double s = 0.;
 #pragma unroll 4
-      for (int64_t t = lane; t < a.tiles; t += 64) v += a.db_part[t * a.E + e];
+      for (int64_t t = lane; t < a.tiles; t += 64) s += double(a.db_part[t * a.E + e]);
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+      const float v = float(s);
       if (lane == 0) {
         if (a.db_bf16) static_cast<uint16_t*>(a.db)[e] = f32_to_bf16(v);
         else static_cast<float*>(a.db)[e] = v;
@@ -642,15 +646,18 @@ __global__ __launch_bounds__(256) void gate_dw_sum_kernel(GateDwSumArgs a) {
   const int64_t n = int64_t(a.E) * a.D, col = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (col >= a.D) return;
   const float* p = a.part + int64_t(blockIdx.y) * a.D + col;
-  v4f v = {0.f, 0.f, 0.f, 0.f};
+  double d4[4] = {0., 0., 0., 0.};
   for (int64_t s = 0; s < a.S; s += 8) {   // eight loads in flight
     v4f u[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) u[j] = *reinterpret_cast<const v4f*>(p + (s + j < a.S ? s + j : s) * n);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (s + j < a.S) v = s + j == 0 ? u[0] : v + u[j];
+      if (s + j < a.S)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d4[i] = s + j == 0 ? double(u[0][i]) : d4[i] + double(u[j][i]);
   }
+  const v4f v = {float(d4[0]), float(d4[1]), float(d4[2]), float(d4[3])};
   const int64_t o = blockIdx.y * a.ld_dw + col;
   if (a.dw_bf16) {
     uint16_t* d = static_cast<uint16_t*>(a.dw) + o;

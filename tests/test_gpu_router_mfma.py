@@ -132,6 +132,27 @@ def test_logits_keep_small_terms_beside_a_large_one(dev, gate):
     assert torch.equal(fm.router_logits(x, w), got)
 
 
+def test_weight_and_bias_gradients_keep_small_terms(dev):
+    """2^25 in the first token, -2^25 in the last: the ones of the token slices between (each slice's own
+    sum is exact) all reach dW, and db has the ones of the large term's own tile of 64 within the 2 that
+    rounding the tile's sum to its ulp of 4 costs."""
+    T, D, E = 16384, 512, 12
+    dl = torch.zeros(T, E, device=dev)
+    x = torch.zeros(T, D, dtype=torch.bfloat16, device=dev)
+    dl[0], dl[1:64], dl[T - 1] = 2.0 ** 25, 1, -(2.0 ** 25)
+    dl[256 + 5:T - 256:256] = 1
+    x[0], x[T - 1] = 1, 1
+    x[256 + 5:T - 256:256] = 1
+    w = torch.zeros(E, D, device=dev)
+    dw, db = torch.empty(E, D, device=dev), torch.empty(E, device=dev)
+    ws = torch.empty(_lib.size_of("fm_router_workspace_bytes", T, D, E), dtype=torch.uint8, device=dev)
+    _lib.call("fm_router_backward", _lib.addr(dl), E, _lib.addr(x), _lib.DTYPE_BF16, D, T, D, _lib.addr(w),
+              _lib.DTYPE_F32, D, E, None, 0, _lib.addr(dw), _lib.DTYPE_F32, D, _lib.addr(db), _lib.DTYPE_F32,
+              _lib.addr(ws), ws.numel(), _lib.stream_of(x))
+    assert torch.all(dw == 62)
+    assert float((db - 125).abs().max()) <= 2
+
+
 @pytest.mark.parametrize("gate", [torch.bfloat16, torch.float32])
 def test_infinite_and_nan_inputs(dev, gate):
     """A non-finite x or gate value reaches the outputs it reaches in fp32 arithmetic, as the same class."""
