@@ -247,8 +247,11 @@ int fm_router_logits(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64_
  * over x plus one small kernel (fm_router_forward_fused says which); other
  * gates with bf16 x take three launches; fp32 x, and gate rows or a workspace off
  * 16-byte boundaries, the steps separately.  T > 0; the workspace holds
- * fm_router_forward_workspace_bytes(T, E) bytes. */
+ * fm_router_forward_workspace_bytes_of(T, D, E, x_dtype, w_dtype) bytes;
+ * fm_router_forward_workspace_bytes(T, E) is enough for every D and dtype (it holds
+ * the chunk sums that the one-pass form has none of). */
 int64_t fm_router_forward_workspace_bytes(int64_t T, int E);
+int64_t fm_router_forward_workspace_bytes_of(int64_t T, int64_t D, int E, int x_dtype, int w_dtype);
 int fm_router_forward_fused(int E, int64_t D, int w_dtype);
 int fm_router_forward(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64_t D, const void* w, int w_dtype,
                       int64_t ld_w, const void* bias, const float* score_bias, int E, int K, int gating, int flags,

@@ -26,6 +26,7 @@
 // differs) except for a small fp32 gate and gate rows off 16-byte boundaries, otherwise
 // as FMAs on the VALU.
 // Gate weights are read as stored (fp32 or bf16).
+#include <algorithm>
 #include <type_traits>
 
 #include "fm_gating.h"
@@ -1195,21 +1196,32 @@ int fm_router_logits(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64_
   return router_logits_launch(a, x_dtype, nullptr, 0, static_cast<hipStream_t>(stream), "fm_router_logits");
 }
 
+// D = 0: whatever D is.
+static int64_t gate_forward_bytes(int64_t T, int64_t D, int E, bool w32) {
+  const GateShape g = gate_shape(T, D, E, w32);
+  return (g.S * T * g.ld_p + gate_blocks(T) * (2 * int64_t(E) + 1)) * 4;
+}
+static int64_t fused_forward_bytes(int64_t T, int E) {
+  const int64_t nb = (T + kRouterRows - 1) / kRouterRows;
+  return nb * (int64_t(E) + 1) * 4 + nb * int64_t(E) * 4;
+}
+static int64_t plain_forward_bytes(int E) { return kRouterForwardWaves * (int64_t(E) + 1) * 4; }
+
 int64_t fm_router_forward_workspace_bytes(int64_t T, int E) {
   if (T <= 0 || E <= 0) return 0;
-  const int64_t nb = (T + kRouterRows - 1) / kRouterRows;
-  const int64_t fused = nb * (int64_t(E) + 1) * 4 + nb * int64_t(E) * 4;
-  const int64_t plain = kRouterForwardWaves * (int64_t(E) + 1) * 4;
-  int64_t most = fused > plain ? fused : plain;
-  if (E <= 256) {
-    const int64_t gb = gate_blocks(T);
-    for (int w32 = 0; w32 < 2; ++w32) {   // the chunk sums and the gating kernel's partials, whatever D is
-      const GateShape g = gate_shape(T, 0, E, w32 != 0);
-      const int64_t b = (g.S * T * g.ld_p + gb * (2 * int64_t(E) + 1)) * 4;
-      most = b > most ? b : most;
-    }
-  }
+  int64_t most = std::max(fused_forward_bytes(T, E), plain_forward_bytes(E));
+  if (E <= 256)
+    for (int w32 = 0; w32 < 2; ++w32) most = std::max(most, gate_forward_bytes(T, 0, E, w32 != 0));
   return most;
+}
+
+int64_t fm_router_forward_workspace_bytes_of(int64_t T, int64_t D, int E, int x_dtype, int w_dtype) {
+  if (T <= 0 || D <= 0 || E <= 0) return 0;
+  const bool w32 = w_dtype != FM_DTYPE_BF16;
+  if (router_small_ok(E, D, !w32)) return fused_forward_bytes(T, E);
+  // (gate rows or a workspace off 16-byte boundaries take the separate steps)
+  if (x_dtype != FM_DTYPE_BF16 || E > 256) return plain_forward_bytes(E);
+  return std::max(plain_forward_bytes(E), gate_forward_bytes(T, D, E, w32));
 }
 
 int fm_router_forward_fused(int E, int64_t D, int w_dtype) {
@@ -1235,8 +1247,9 @@ int fm_router_forward(const void* x, int x_dtype, int64_t ld_x, int64_t T, int64
   FM_REQUIRE((tokens_per_expert == nullptr) == (total_tokens == nullptr),
              "fm_router_forward: tokens_per_expert and total_tokens go together");
   FM_REQUIRE(T > 0, "fm_router_forward: T must be positive (the loss divides by it)");
-  FM_REQUIRE(workspace != nullptr && workspace_bytes >= fm_router_forward_workspace_bytes(T, E),
-             "fm_router_forward: workspace of fm_router_forward_workspace_bytes(T, E) bytes required");
+  FM_REQUIRE(workspace != nullptr && workspace_bytes >= fm_router_forward_workspace_bytes_of(T, D, E, x_dtype, w_dtype),
+             "fm_router_forward: workspace of fm_router_forward_workspace_bytes_of(T, D, E, x_dtype, w_dtype) bytes "
+             "required");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RouterArgs a{x, ld_x, T, D, w, ld_w, bias, w_dtype == FM_DTYPE_BF16, score_bias, E, logits, ld_l};
   const int sigmoid = gating == FM_GATING_SIGMOID;

@@ -380,7 +380,8 @@ def router_forward(x2, gate_weight, gate_bias, score_bias, top_k, gating, replay
     idx = torch.empty(T, K, dtype=torch.int64, device=dev)
     counts = torch.empty(E, dtype=torch.int32, device=dev)
     aux = torch.empty((), dtype=torch.float32, device=dev)
-    ws = torch.empty(_lib.size_of("fm_router_forward_workspace_bytes", T, E), dtype=torch.uint8, device=dev)
+    ws = torch.empty(_lib.size_of("fm_router_forward_workspace_bytes_of", T, D, E, _x_dtype(x2), _dt_code(w_)),
+                     dtype=torch.uint8, device=dev)
     rep = None
     if replay is not None:
         rep = replay.reshape(T, K)
