@@ -576,7 +576,8 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
         elif w.paired:
             raise ValueError("paired-row weights need paired-row tokens")
         if (t_paired or kind == _lib.QUANT_BF16) and _m_split(kind, plan, w, out, mask):
-            ws = torch.empty(_cus(out.device) * _SLICE_BYTES, dtype=torch.uint8, device=out.device)
+            ws = torch.empty(_slice_slots(kind, plan, w, _cus(out.device)) * _SLICE_BYTES, dtype=torch.uint8,
+                             device=out.device)
             _lib.call("fm_grouped_gemm_ragged_m_split", gk, _token_operand(tokens, kind), w.operand(), plan.m_tiles,
                       _lib.addr(plan.tile_expert), _lib.addr(plan.offsets), plan.num_experts, w.N, w.K,
                       _lib.addr(mask), want, _lib.addr(out), out.stride(0), _lib.addr(ws), ws.numel(),
@@ -595,6 +596,17 @@ def _gemm_m(kind, tokens, w: ExpertWeightOperand, plan: RoutingPlan, out, mask=N
 
 # A slice's fp32 partial of a 256 x 256 tile (fm_grouped_gemm_ragged_m_split).
 _SLICE_BYTES = 256 << 10
+
+
+def _slice_slots(kind, plan: RoutingPlan, w: ExpertWeightOperand, cus: int) -> int:
+    """Partials that a sliced launch can write: one per workgroup, and no more workgroups
+    than the most tiles (of the plan's rows, in whole rounds of the 8 XCDs) have slices (8, of
+    at least 8 K steps); with as many, the device's choice of slices is that with all CUs."""
+    tiles = (plan.m_tiles + plan.num_experts + 1) // 2 * -(-w.N // 256)
+    nk = w.K // (64 if kind == _lib.QUANT_BF16 else 128)
+    return min(cus, -(-tiles // 8) * 8 * min(8, nk // 8))
+
+
 _SLICE_GAIN = 5.25   # K steps (about 6 us) that slicing must save by the model
 
 

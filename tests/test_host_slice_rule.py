@@ -5,16 +5,24 @@ the largest of equals."""
 
 import ctypes
 import subprocess
+import types
 from fractions import Fraction
+from itertools import product
 from pathlib import Path
 
 import pytest
+
+import nanopysche_amd.flow_moe as fmm
+from nanopysche_amd import _lib
 
 CSRC = Path(__file__).resolve().parents[1] / "nanopysche_amd" / "csrc"
 SOURCE = f"""
 #include "{CSRC / 'fm_slices.h'}"
 extern "C" void counts(int nk, int bf16, int tiles, int* out) {{   // of 1 .. tiles tiles, 32 workgroups an XCD
   for (int n = 1; n <= tiles; ++n) out[n - 1] = fm::slice_count(n, 32 / ((n + 7) / 8), nk, bf16 != 0);
+}}
+extern "C" int count(int nk, int bf16, int tiles, int workgroups) {{
+  return fm::slice_count(tiles, workgroups / 8 / ((tiles + 7) / 8), nk, bf16 != 0);
 }}
 """
 
@@ -58,3 +66,23 @@ def test_counts_of_equal_cost(built):
     """BF16, 16 tiles of 64 steps and 32 of 128: 7 and 8 slices cost the same."""
     for nk, tiles in ((64, 16), (128, 32)):
         assert [_counts(lib, nk, True)[tiles - 1] for lib in built] == [8, 8]
+
+
+@pytest.mark.parametrize("kind", [_lib.QUANT_BF16, _lib.QUANT_POW2])
+def test_the_workspace_does_not_change_the_count(built, kind):
+    """With the slots that the host allocates (a workgroup each), every number of tiles that the
+    plan can hold gets the slices that 256 workgroups would give it, in as many slots."""
+    bf16 = kind == _lib.QUANT_BF16
+    sizes = set()
+    for E, tokens, N, steps in product((1, 4, 8), (64, 200, 700), (256, 384, 1024, 4096), (20, 34, 64, 88, 224)):
+        m_tiles = -(-tokens // 128) + E
+        plan = types.SimpleNamespace(m_tiles=m_tiles, num_experts=E)
+        w = types.SimpleNamespace(N=N, K=steps * (64 if bf16 else 128))
+        slots = fmm._slice_slots(kind, plan, w, 256)
+        sizes.add(slots)
+        assert slots % 8 == 0 and slots <= 256
+        for tiles in range(1, min(256, (m_tiles + E + 1) // 2 * -(-N // 256)) + 1):
+            n = built[0].count(steps, int(bf16), tiles, slots)
+            assert n == built[0].count(steps, int(bf16), tiles, 256)
+            assert n == 1 or -(-tiles // 8) * 8 * n <= slots
+    assert min(sizes) == 16 and max(sizes) == 256
