@@ -1313,6 +1313,7 @@ class FP8FlowMoECompute:
         {"addend": bf16 [T, D]}, or with ``can_fold`` {"dlogits": [T, E],
         "gate_w": [E, D]} (E <= 8) for the unpermute to form it itself."""
         wts, GU, Y = ctx.saved_tensors
+        wts = wts.to(torch.float32).contiguous()   # as saved, unless a saved-tensor hook returned it otherwise
         if any(w._version != version for w, version in ctx.in_place):
             raise RuntimeError("expert weights that the backward reads in place (BF16) were changed by an in-place "
                                "operation after the forward")
@@ -1397,7 +1398,7 @@ class FP8FlowMoECompute:
         for kind, want in runs:
             dgu_row, dgu_col, args = _alloc_act(R, 2 * H, kind, True, dev, self._paired(kind), pcols.get(kind, False))
             gu = GU.data_ptr()
-            _lib.call("fm_swiglu_backward", gu, 2 * H, gu + 2 * H, 2 * H, dH.data_ptr(), H, R, H, *args,
+            _lib.call("fm_swiglu_backward", gu, GU.stride(0), gu + 2 * H, GU.stride(0), dH.data_ptr(), H, R, H, *args,
                       _lib.ptr(tiles.get(kind, plan.tile_expert)), _lib.stream_of(GU))
             # dW1 | dW3: contraction over each expert's tokens
             _gemm_k(kind, dgu_col, ctx.saved_cols[kind], plan, 2 * H, D, dW1, H * D, dW3, H * D, split=H,
