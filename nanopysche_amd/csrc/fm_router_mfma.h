@@ -15,9 +15,10 @@
 //
 // Measured on MI355X for [4096, 7168] bf16 x and a bf16 gate of 256 experts,
 // against FMAs on the VALU (15 GFLOP a product, bound by their issue): logits
-// 574 -> 38 us, gating + counts + loss 187 -> 32, dx 1167 -> 64, dw 380 -> 75, the pieces
-// themselves 12.  What bounds them now: the logits x's read and the chunk sums'
-// write and read (floor 10 us of HBM), dx and dw their 45 GFLOP of pieces at
+// 574 -> 49 us, gating + counts + loss 187 -> 29, dx 1167 -> 63, dw 380 -> 75, the pieces
+// themselves 13.  What bounds them now: the logits x's read, the chunk sums'
+// write and read (floor 10 us of HBM) and the joins of the MFMA chains' sums (10 us), dx
+// and dw their 45 GFLOP of pieces at
 // 0.7 PFLOP/s, fragments fetched from the L2.
 #pragma once
 
@@ -193,7 +194,8 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void gate_logits_kernel(GateLog
           }
         }
       }
-      // the group's sums into the chunk's; what that rounding drops starts the next group's
+      // the chain's sums into the chunk's; what that rounding drops starts the next chain
+      // (nothing where a sum is not finite)
       if (((k - k0) & a.group) != a.group && k + 64 < k1) continue;
 #pragma unroll
       for (int f = 0; f < NF; ++f)
@@ -245,14 +247,17 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void gate_logits_kernel(GateLog
 // The launch's shape: fragments per wave, chunks of D.  About 2048 waves (two
 // per SIMD, which is what hides the fragments' latency) where D allows chunks
 // of at least 128 columns; more chunks would only add partial sums to write
-// and read (4 bytes of part per token, expert and chunk).
+// and read (4 bytes of part per token, expert and chunk).  The tile leaves two waves
+// a SIMD their registers: two sums per output, three with an fp32 gate ([4096, 7168] x 256,
+// bf16 gate: 64 x 64 outputs 89 us, 76 with the registers of two waves and spills, 32 x 64 72;
+// fp32 gate: 32 x 64 279 and 210, 32 x 32 176).
 struct GateShape {
   int tf, nf, eg;
   int64_t tt, S, chunk, ld_p;
 };
 inline GateShape gate_shape(int64_t T, int64_t D, int E, bool w32) {
   GateShape g;
-  g.nf = E <= 16 ? 1 : E <= 32 || w32 ? 2 : E <= 48 ? 3 : 4;   // an fp32 gate: two sums per output
+  g.nf = E <= 16 ? 1 : E <= 32 || w32 ? 2 : E <= 48 ? 3 : 4;
   g.tf = T <= 16 ? 1 : (T <= 32 || w32 || g.nf == 4) ? 2 : 4;
   g.eg = (E + 16 * g.nf - 1) / (16 * g.nf);
   g.tt = (T + 16 * g.tf - 1) / (16 * g.tf);
@@ -270,12 +275,12 @@ inline GateShape gate_shape(int64_t T, int64_t D, int E, bool w32) {
   return g;
 }
 
-// Columns of an MFMA chain: short enough that the rms error is below the FMA
-// kernel's at every D.  FMAs, chains of 64, 128 and 256 columns, bf16 gate (16384
-// tokens): D 384 5.9e-8, 5.7e-8, (chunk) 6.9e-8; 1024 6.8e-8, 5.7e-8, 7.0e-8; 4096 8.4e-8,
-// 5.8e-8, 7.1e-8, 9.4e-8; fp32 gate: D 512 8.6e-8, 5.7e-8, 6.9e-8, 9.0e-8; 2560 1.3e-7, 5.7e-8, 7e-8, 9e-8.
-// A join is five VALU instructions a sum: forward of [4096, 7168] x 256 with 64 / 128 / 256
-// columns 80 / 75 / 72 us.
+// Columns of an MFMA chain: the longest that leaves the rms error below the FMA kernel's
+// (16384 tokens, in units of the logits').  bf16 gate, FMAs | chains of 64 / 128 / 256 columns:
+// D 512 6.1e-8 | 5.7e-8 / 7.2e-8 / -, D 1024 6.8e-8 | 5.7e-8, D 2048 7.5e-8 | 5.8e-8 / 7.0e-8 / -, D 4096
+// 8.4e-8 | 5.8e-8 / 7.1e-8 / 9.4e-8.  fp32 gate: D 512 8.6e-8 | 5.7e-8 / 6.9e-8 / 9.0e-8, D 2560 1.3e-7 |
+// 5.7e-8 / - / 8.9e-8.  A join is five VALU instructions a sum: forward of [4096, 7168] x 256 with
+// 64 / 128 / 256 columns 80 / 75 / 72 us.
 inline int gate_group_columns(int64_t D, bool w32) { return (D < 2048 ? 64 : 128) << int(w32); }
 
 // ------------------------------------------- pieces for the backward ----
